@@ -1,0 +1,30 @@
+// Control block of the generic-graph solve kernel (csr_kernels.h), shared with its host driver.
+#pragma once
+
+#include <cstdint>
+
+namespace cgp {
+
+enum CsrStatus : int32_t { kCsrRunning = 0, kCsrDone = 1, kCsrNotConverged = 2 };
+enum CsrGate : int32_t { kCsrGateOpen = 1, kCsrGateClosed = 2 };
+
+// Stages of a launch. A plain solve runs all of them until it is done; with trace hooks the host
+// launches a relabel and the push steps that follow it one at a time.
+enum CsrStage : int32_t { kCsrRelabel = 1, kCsrPush = 2, kCsrLoop = 4, kCsrClosure = 8 };
+
+// Device control block; every phase (barrier interval) uses word phase % 3: low half the workgroups
+// that arrived, high half the entries appended to the list under construction. The word of the
+// next phase is cleared by workgroup 0 during a phase: it was last read two barriers before.
+struct CsrControl {
+	unsigned long long word[3];
+	unsigned long long flow;
+	int32_t active[2];   // length of the active list a relabel builds, by round parity
+	int32_t list_count;  // active vertices after the last relabel
+	int32_t levels;      // levels of the last relabel (queue ends in starts[1 .. levels])
+	int32_t rounds, status, threshold;
+	int32_t arrived, gate;  // workgroups that started; whether the launch runs
+	int32_t solo[4];     // what workgroup 0 left after running short steps alone
+	long long bfs_passes, push_steps, cut_passes;
+};
+
+}  // namespace cgp

@@ -5,299 +5,24 @@
 //
 //   relabel: level-synchronous BFS from the sink frontier (level 1 = residual sink link)
 //            over reverse residual edges, vertices appended to one queue in level order
-//            (initBFSKernel, propagateFromVertex, bfs_iteration / bfs_multi_iteration,
-//            graph_cut_relabeling.hpp:47-112, 1004-1240);
-//   push:    levels from the top down to 1, every vertex of the level pushing to any neighbour
-//            with a lower label, level 1 also into t (pushImplementation / PushIteration,
-//            graph_cut_push.hpp:160-186, 395-482);
-//   loop:    until a sweep pushes nothing (MinCut::compute, graph_cut_implementation.hpp:122-198).
-// Small levels run inside one workgroup for many levels per launch, like the reference's
-// single-block multi-level kernels.
+//            (initBFSKernel, propagateFromVertex, graph_cut_relabeling.hpp:47-112, 1004-1240);
+//   push:    synchronous push/relabel steps over the vertices that hold excess: each pushes into t
+//            and along its arcs to neighbours one label lower (pushImplementation,
+//            graph_cut_push.hpp:160-186, 395-482) and, if excess is left, raises its own label;
+//   loop:    until a relabel finds no vertex with excess that reaches t (MinCut::compute,
+//            graph_cut_implementation.hpp:122-198).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
 
 #include "common.h"
+#include "csr_kernels.h"
 #include "solver.h"
 
 namespace cgp {
 
 namespace {
-
-constexpr int kMultiLevelLimit = 4096;   // level size handled by the single-workgroup kernels
-constexpr int kMultiLevelThreads = 1024;
-constexpr int kMaxLevelsPerLaunch = 1024;
-
-__global__ __launch_bounds__(256) void k_csr_init_vertices(int n, const int32_t *cs, const int32_t *ct, int32_t *e,
-                                                           int32_t *rt)
-{
-	for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-		e[v] = cs[v];
-		rt[v] = ct[v];
-	}
-}
-
-__global__ __launch_bounds__(256) void k_csr_copy(int64_t n, const int32_t *src, int32_t *dst)
-{
-	for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-		dst[i] = src[i];
-	}
-}
-
-// Append every vertex satisfying `pred` to queue (one atomic per wave).
-__device__ inline void wave_append(bool pred, int v, int32_t *queue, int32_t *tail)
-{
-	const unsigned long long ballot = __ballot(pred);
-	const int lane = threadIdx.x & 63;
-	int base = 0;
-	if (lane == 0 && ballot) {
-		base = atomicAdd(tail, (int)__popcll(ballot));
-	}
-	base = __shfl(base, 0, 64);
-	if (pred) {
-		queue[base + (int)__popcll(ballot & ((1ull << lane) - 1ull))] = v;
-	}
-}
-
-// Level 1 of the BFS: vertices whose sink link still has residual capacity.
-__global__ __launch_bounds__(256) void k_csr_bfs_seed(int n, const int32_t *rt, int32_t threshold, int32_t *h,
-                                                      int32_t *queue, int32_t *tail)
-{
-	const int stride = gridDim.x * blockDim.x;
-	const int start = blockIdx.x * blockDim.x + threadIdx.x;
-	// whole waves iterate together so that the ballot sees every lane
-	const int rounds = (n + stride - 1) / stride;
-	for (int r = 0; r < rounds; ++r) {
-		const int v = start + r * stride;
-		bool seed = false;
-		if (v < n) {
-			seed = rt[v] > threshold;
-			h[v] = seed ? 1 : kLabelInf;
-		}
-		wave_append(seed, v, queue, tail);
-	}
-}
-
-// Append v to queue where pred holds, among the lanes active at the call (also inside loops whose
-// trip counts differ per lane): the lowest active lane reserves the entries of the whole wave with
-// one atomic, and each lane stores at its rank.
-__device__ inline void wave_append_active(bool pred, int v, int32_t *queue, int32_t *tail)
-{
-	const unsigned long long active = __ballot(1);
-	const unsigned long long ballot = __ballot(pred);
-	if (!ballot) {
-		return;  // (the same for every active lane)
-	}
-	const int lane = threadIdx.x & 63;
-	const int leader = __ffsll((long long)active) - 1;
-	int base = 0;
-	if (lane == leader) {
-		base = atomicAdd(tail, (int)__popcll(ballot));
-	}
-	base = __shfl(base, leader, 64);
-	if (pred) {
-		queue[base + (int)__popcll(ballot & ((1ull << lane) - 1ull))] = v;
-	}
-}
-
-// Label the unlabelled neighbours u of frontier vertex v that can reach v (residual u -> v > threshold).
-__device__ inline void expand_towards_sink(int v, int32_t level, const int32_t *first, const int32_t *head,
-                                           const int32_t *mate, const int32_t *res, int32_t threshold, int32_t *h,
-                                           int32_t *queue, int32_t *tail)
-{
-	for (int a = first[v]; a < first[v + 1]; ++a) {
-		const int u = head[a];
-		bool claimed = false;
-		if (h[u] == kLabelInf && res[mate[a]] > threshold) {
-			claimed = atomicCAS(&h[u], kLabelInf, level + 1) == kLabelInf;
-		}
-		wave_append_active(claimed, u, queue, tail);
-	}
-}
-
-// The flow into t is summed in kSlots slots on separate cache lines, picked by workgroup: one
-// word taking an atomic from every workgroup serialises them in the L2.
-constexpr int kFlowSlots = 32;
-constexpr int kFlowSlotStride = 16;
-
-__device__ inline void add_flow(unsigned long long *flow, long long total)
-{
-	if (total) {
-		atomicAdd(flow + (blockIdx.x & (kFlowSlots - 1)) * kFlowSlotStride, (unsigned long long)total);
-	}
-}
-
-__global__ void k_csr_sum_flow(const unsigned long long *slots, unsigned long long *total)
-{
-	if (threadIdx.x == 0 && blockIdx.x == 0) {
-		unsigned long long sum = 0;
-		for (int j = 0; j < kFlowSlots; ++j) {
-			sum += slots[j * kFlowSlotStride];
-		}
-		*total = sum;
-	}
-}
-
-__global__ __launch_bounds__(256) void k_csr_bfs_level(int32_t qs, int32_t qe, int32_t level, const int32_t *first,
-                                                       const int32_t *head, const int32_t *mate, const int32_t *res,
-                                                       int32_t threshold, int32_t *h, int32_t *queue, int32_t *tail)
-{
-	for (int i = qs + blockIdx.x * blockDim.x + threadIdx.x; i < qe; i += gridDim.x * blockDim.x) {
-		expand_towards_sink(queue[i], level, first, head, mate, res, threshold, h, queue, tail);
-	}
-}
-
-// Many small BFS levels in one workgroup. Writes the queue end after each level to starts[] and
-// the number of levels processed to *levels_out.
-__global__ __launch_bounds__(kMultiLevelThreads) void k_csr_bfs_multi(int32_t qs, int32_t qe, int32_t level,
-                                                                      const int32_t *first, const int32_t *head,
-                                                                      const int32_t *mate, const int32_t *res,
-                                                                      int32_t threshold, int32_t *h, int32_t *queue,
-                                                                      int32_t *tail, int32_t *starts,
-                                                                      int32_t *levels_out)
-{
-	int done = 0;
-	for (;;) {
-		for (int i = qs + (int)threadIdx.x; i < qe; i += blockDim.x) {
-			expand_towards_sink(queue[i], level, first, head, mate, res, threshold, h, queue, tail);
-		}
-		__syncthreads();
-		const int32_t nt = atomicAdd(tail, 0);
-		if (threadIdx.x == 0) {
-			starts[done] = nt;
-		}
-		++done;
-		__syncthreads();
-		if (nt == qe || nt - qe > kMultiLevelLimit || done >= kMaxLevelsPerLaunch) {
-			break;
-		}
-		qs = qe;
-		qe = nt;
-		++level;
-	}
-	if (threadIdx.x == 0) {
-		*levels_out = done;
-	}
-}
-
-__device__ inline bool push_vertex(int v, int32_t level, const int32_t *first, const int32_t *head,
-                                   const int32_t *mate, int32_t *res, int32_t *e, int32_t *rt, const int32_t *h,
-                                   long long &sink)
-{
-	int32_t ex = e[v];
-	if (ex <= 0) {
-		return false;
-	}
-	bool pushed = false;
-	if (rt[v] > 0) {
-		const int32_t f = ex < rt[v] ? ex : rt[v];
-		rt[v] -= f;
-		ex -= f;
-		sink += f;
-		pushed = true;
-	}
-	for (int a = first[v]; a < first[v + 1] && ex > 0; ++a) {
-		const int u = head[a];
-		const int32_t hu = h[u];
-		const int32_t rv = res[a];
-		if (hu < level && rv > 0) {
-			const int32_t f = ex < rv ? ex : rv;
-			res[a] = rv - f;
-			res[mate[a]] += f;   // only v pushes along this edge during this level
-			atomicAdd(&e[u], f); // several vertices of the level may feed u
-			ex -= f;
-			pushed = true;
-		}
-	}
-	e[v] = ex;
-	return pushed;
-}
-
-__global__ __launch_bounds__(256) void k_csr_push_level(int32_t qs, int32_t qe, int32_t level, const int32_t *queue,
-                                                        const int32_t *first, const int32_t *head,
-                                                        const int32_t *mate, int32_t *res, int32_t *e, int32_t *rt,
-                                                        const int32_t *h, unsigned long long *flow, int32_t *pushed)
-{
-	__shared__ long long red[4];
-	long long sink = 0;
-	bool any = false;
-	for (int i = qs + blockIdx.x * blockDim.x + threadIdx.x; i < qe; i += gridDim.x * blockDim.x) {
-		any |= push_vertex(queue[i], level, first, head, mate, res, e, rt, h, sink);
-	}
-	if (any) {
-		*pushed = 1;
-	}
-	const long long total = block_sum_i64<256>(sink, red);
-	if (threadIdx.x == 0) {
-		add_flow(flow, total);
-	}
-}
-
-// Consecutive small levels, from `level` downwards, in one workgroup; stops at level 0 or at the
-// first level above the size limit. Writes the first level not processed to *next_level.
-__global__ __launch_bounds__(kMultiLevelThreads) void k_csr_push_multi(int32_t level, const int32_t *starts,
-                                                                       const int32_t *queue, const int32_t *first,
-                                                                       const int32_t *head, const int32_t *mate,
-                                                                       int32_t *res, int32_t *e, int32_t *rt,
-                                                                       const int32_t *h, unsigned long long *flow,
-                                                                       int32_t *pushed, int32_t *next_level)
-{
-	__shared__ long long red[kMultiLevelThreads / 64];
-	long long sink = 0;
-	bool any = false;
-	while (level >= 1) {
-		const int32_t qs = starts[level - 1], qe = starts[level];
-		if (qe - qs > kMultiLevelLimit) {
-			break;
-		}
-		for (int i = qs + (int)threadIdx.x; i < qe; i += blockDim.x) {
-			any |= push_vertex(queue[i], level, first, head, mate, res, e, rt, h, sink);
-		}
-		__syncthreads();
-		--level;
-	}
-	if (any) {
-		*pushed = 1;
-	}
-	const long long total = block_sum_i64<kMultiLevelThreads>(sink, red);
-	if (threadIdx.x == 0) {
-		add_flow(flow, total);
-		*next_level = level;
-	}
-}
-
-// S_min closure: mark vertices with excess, then everything reachable over residual arcs.
-__global__ __launch_bounds__(256) void k_csr_closure_seed(int n, const int32_t *e, int32_t *mark, int32_t *queue,
-                                                          int32_t *tail)
-{
-	const int stride = gridDim.x * blockDim.x;
-	const int start = blockIdx.x * blockDim.x + threadIdx.x;
-	const int rounds = (n + stride - 1) / stride;
-	for (int r = 0; r < rounds; ++r) {
-		const int v = start + r * stride;
-		bool seed = false;
-		if (v < n) {
-			seed = e[v] > 0;
-			mark[v] = seed ? 1 : 0;
-		}
-		wave_append(seed, v, queue, tail);
-	}
-}
-
-__global__ __launch_bounds__(256) void k_csr_closure_level(int32_t qs, int32_t qe, const int32_t *first,
-                                                           const int32_t *head, const int32_t *res, int32_t *mark,
-                                                           int32_t *queue, int32_t *tail)
-{
-	for (int i = qs + blockIdx.x * blockDim.x + threadIdx.x; i < qe; i += gridDim.x * blockDim.x) {
-		const int v = queue[i];
-		for (int a = first[v]; a < first[v + 1]; ++a) {
-			const int u = head[a];
-			const bool claimed = res[a] > 0 && mark[u] == 0 && atomicCAS(&mark[u], 0, 1) == 0;
-			wave_append_active(claimed, u, queue, tail);
-		}
-	}
-}
 
 __global__ __launch_bounds__(256) void k_csr_masks(int n, const int32_t *h, const int32_t *mark, uint8_t *out,
                                                    int mode, uint8_t mask, uint8_t background)
@@ -342,17 +67,16 @@ void CsrSolver::set_vertex_count(int n)
 	mRt.allocate(n);
 	mH.allocate(n);
 	mQueue.allocate(n);
+	mList[0].allocate(n);
+	mList[1].allocate(n);
 	mS.allocate(n);
-	mTail.allocate(1);
-	mPushed.allocate(1);
-	mStatus.allocate(1);
-	mLevelStarts.allocate(kMaxLevelsPerLaunch + 2);
-	mFlow.allocate(kFlowSlots * kFlowSlotStride + 1);  // slots, then their sum
-	mPinned.allocate(kMaxLevelsPerLaunch + 8);
-	mHead.release();
-	mMate.release();
-	mArcCap.release();
-	mRes.release();
+	mMask.allocate(n);
+	mLevelStarts.allocate((size_t)n + 2);
+	mControl.allocate(1);
+	mPinned.allocate(1);
+	mEnds.release();
+	mCap.release();
+	mPair.release();
 	CGP_HIP(hipStreamSynchronize(mStream));
 }
 
@@ -392,7 +116,7 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 	}
 	const int64_t arcs = first[mN];
 	std::vector<int32_t> pos(first.begin(), first.end() - 1);
-	std::vector<int32_t> head(arcs), mate(arcs), cap(arcs);
+	std::vector<int2> ends(arcs), cap(arcs);  // {head, mate}, {capacity, the mate's capacity}
 	std::vector<int64_t> incoming(mN, 0);
 	for (int i = 0; i < m; ++i) {
 		const int a = (int)edges[i].first, b = (int)edges[i].second;
@@ -400,12 +124,10 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 			continue;
 		}
 		const int ia = pos[a]++, ib = pos[b]++;
-		head[ia] = b;
-		cap[ia] = fwd[i];
-		mate[ia] = ib;
-		head[ib] = a;
-		cap[ib] = bwd[i];
-		mate[ib] = ia;
+		ends[ia] = make_int2(b, ib);
+		cap[ia] = make_int2(fwd[i], bwd[i]);
+		ends[ib] = make_int2(a, ia);
+		cap[ib] = make_int2(bwd[i], fwd[i]);
 		incoming[b] += fwd[i];
 		incoming[a] += bwd[i];
 	}
@@ -413,16 +135,15 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 	mHostFirst.swap(first);
 	mArcs = arcs;
 	mSolved = false;
+	mHeadroomChecked = false;
 	mFirst.allocate(mN + 1);
 	CGP_HIP(hipMemcpyAsync(mFirst.get(), mHostFirst.data(), (mN + 1) * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
 	if (arcs > 0) {
-		mHead.allocate(arcs);
-		mMate.allocate(arcs);
-		mArcCap.allocate(arcs);
-		mRes.allocate(arcs);
-		CGP_HIP(hipMemcpyAsync(mHead.get(), head.data(), arcs * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
-		CGP_HIP(hipMemcpyAsync(mMate.get(), mate.data(), arcs * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
-		CGP_HIP(hipMemcpyAsync(mArcCap.get(), cap.data(), arcs * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
+		mEnds.allocate(arcs);
+		mCap.allocate(arcs);
+		mPair.allocate(arcs);
+		CGP_HIP(hipMemcpyAsync(mEnds.get(), ends.data(), arcs * sizeof(int2), hipMemcpyHostToDevice, mStream));
+		CGP_HIP(hipMemcpyAsync(mCap.get(), cap.data(), arcs * sizeof(int2), hipMemcpyHostToDevice, mStream));
 	}
 	CGP_HIP(hipStreamSynchronize(mStream));
 }
@@ -445,6 +166,7 @@ void CsrSolver::set_tweights(const int32_t *source, const int32_t *sink)
 	CGP_HIP(hipMemcpyAsync(mCt.get(), sink, mN * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
 	CGP_HIP(hipStreamSynchronize(mStream));
 	mHaveTweights = true;
+	mHeadroomChecked = false;
 	mSolved = false;
 }
 
@@ -454,10 +176,10 @@ void CsrSolver::export_graph(std::vector<int32_t> &tail, std::vector<int32_t> &h
 	if (!ready()) {
 		fail(CGP_ERR_STATE, "no complete graph set");
 	}
-	std::vector<int32_t> heads((size_t)mArcs), caps((size_t)mArcs);
+	std::vector<int2> ends((size_t)mArcs), caps((size_t)mArcs);
 	if (mArcs) {
-		CGP_HIP(hipMemcpyAsync(heads.data(), mHead.get(), mArcs * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
-		CGP_HIP(hipMemcpyAsync(caps.data(), mArcCap.get(), mArcs * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
+		CGP_HIP(hipMemcpyAsync(ends.data(), mEnds.get(), mArcs * sizeof(int2), hipMemcpyDeviceToHost, mStream));
+		CGP_HIP(hipMemcpyAsync(caps.data(), mCap.get(), mArcs * sizeof(int2), hipMemcpyDeviceToHost, mStream));
 	}
 	cs.resize((size_t)mN);
 	ct.resize((size_t)mN);
@@ -469,125 +191,84 @@ void CsrSolver::export_graph(std::vector<int32_t> &tail, std::vector<int32_t> &h
 	cap.clear();
 	for (int v = 0; v < mN; ++v) {
 		for (int a = mHostFirst[(size_t)v]; a < mHostFirst[(size_t)v + 1]; ++a) {
-			if (caps[(size_t)a] > 0) {
+			if (caps[(size_t)a].x > 0) {
 				tail.push_back(v);
-				head.push_back(heads[(size_t)a]);
-				cap.push_back(caps[(size_t)a]);
+				head.push_back(ends[(size_t)a].x);
+				cap.push_back(caps[(size_t)a].x);
 			}
 		}
 	}
 }
 
-int64_t CsrSolver::read_flow()
+// Runs `stages` of the solve kernel and reads the control block back.
+const CsrControl &CsrSolver::run_stages(int32_t stages, int32_t max_rounds)
 {
-	unsigned long long *total = mFlow.get() + kFlowSlots * kFlowSlotStride;
-	hipLaunchKernelGGL(k_csr_sum_flow, dim3(1), dim3(64), 0, mStream, (const unsigned long long *)mFlow.get(), total);
-	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipMemcpyAsync(mPinned.get(), total, sizeof(unsigned long long), hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
-	int64_t f;
-	std::memcpy(&f, mPinned.get(), sizeof(f));
-	return f;
-}
-
-int32_t CsrSolver::read_i32(const int32_t *device_ptr)
-{
-	CGP_HIP(hipMemcpyAsync(mPinned.get(), device_ptr, sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
-	return mPinned[0];
-}
-
-int CsrSolver::bfs(int32_t threshold, std::vector<int32_t> &level_starts, cgp_stats &stats)
-{
-	CGP_HIP(hipMemsetAsync(mTail.get(), 0, sizeof(int32_t), mStream));
-	hipLaunchKernelGGL(k_csr_bfs_seed, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mRt.get(), threshold, mH.get(),
-	                   mQueue.get(), mTail.get());
-	CGP_LAUNCH_CHECK();
-	level_starts.assign(1, 0);
-	level_starts.push_back(read_i32(mTail.get()));
-	int level = 1;
-	while (level_starts[level] > level_starts[level - 1]) {
-		const int32_t qs = level_starts[level - 1], qe = level_starts[level];
-		if (qe - qs <= kMultiLevelLimit) {
-			hipLaunchKernelGGL(k_csr_bfs_multi, dim3(1), dim3(kMultiLevelThreads), 0, mStream, qs, qe, level, mFirst.get(),
-			                   mHead.get(), mMate.get(), mRes.get(), threshold, mH.get(), mQueue.get(), mTail.get(),
-			                   mLevelStarts.get(), mLevelStarts.get() + kMaxLevelsPerLaunch + 1);
-			CGP_LAUNCH_CHECK();
-			CGP_HIP(hipMemcpyAsync(mPinned.get(), mLevelStarts.get(), (kMaxLevelsPerLaunch + 2) * sizeof(int32_t),
-			                       hipMemcpyDeviceToHost, mStream));
-			CGP_HIP(hipStreamSynchronize(mStream));
-			const int done = mPinned[kMaxLevelsPerLaunch + 1];
-			stats.bfs_passes += done;
-			for (int i = 0; i < done; ++i) {
-				const int32_t nt = mPinned[i];
-				if (nt == level_starts.back()) {
-					return (int)level_starts.size() - 1;
-				}
-				level_starts.push_back(nt);
-				++level;
-			}
-		} else {
-			hipLaunchKernelGGL(k_csr_bfs_level, dim3(grid_blocks(qe - qs)), dim3(256), 0, mStream, qs, qe, level,
-			                   mFirst.get(), mHead.get(), mMate.get(), mRes.get(), threshold, mH.get(), mQueue.get(),
-			                   mTail.get());
-			CGP_LAUNCH_CHECK();
-			++stats.bfs_passes;
-			const int32_t nt = read_i32(mTail.get());
-			if (nt == qe) {
-				break;
-			}
-			level_starts.push_back(nt);
-			++level;
-		}
-	}
-	return (int)level_starts.size() - 1;
-}
-
-bool CsrSolver::push_sweep(const std::vector<int32_t> &level_starts, cgp_stats &stats)
-{
-	const int top = (int)level_starts.size() - 1;
-	DeviceBuffer<int32_t> starts(level_starts.size());
-	CGP_HIP(hipMemcpyAsync(starts.get(), level_starts.data(), level_starts.size() * sizeof(int32_t),
-	                       hipMemcpyHostToDevice, mStream));
-	CGP_HIP(hipMemsetAsync(mPushed.get(), 0, sizeof(int32_t), mStream));
-	int level = top;
-	while (level >= 1) {
-		const int32_t qs = level_starts[level - 1], qe = level_starts[level];
-		if (qe - qs <= kMultiLevelLimit) {
-			hipLaunchKernelGGL(k_csr_push_multi, dim3(1), dim3(kMultiLevelThreads), 0, mStream, level, starts.get(),
-			                   mQueue.get(), mFirst.get(), mHead.get(), mMate.get(), mRes.get(), mE.get(), mRt.get(),
-			                   mH.get(), mFlow.get(), mPushed.get(), mStatus.get());
-			CGP_LAUNCH_CHECK();
-			const int next = read_i32(mStatus.get());
-			stats.discharge_phases += level - next;
-			level = next;
-		} else {
-			hipLaunchKernelGGL(k_csr_push_level, dim3(grid_blocks(qe - qs)), dim3(256), 0, mStream, qs, qe, level,
-			                   mQueue.get(), mFirst.get(), mHead.get(), mMate.get(), mRes.get(), mE.get(), mRt.get(),
-			                   mH.get(), mFlow.get(), mPushed.get());
-			CGP_LAUNCH_CHECK();
-			++stats.discharge_phases;
-			--level;
-		}
-	}
-	return read_i32(mPushed.get()) != 0;
-}
-
-void CsrSolver::source_closure(cgp_stats &stats)
-{
-	CGP_HIP(hipMemsetAsync(mTail.get(), 0, sizeof(int32_t), mStream));
-	hipLaunchKernelGGL(k_csr_closure_seed, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mE.get(), mS.get(),
-	                   mQueue.get(), mTail.get());
-	CGP_LAUNCH_CHECK();
-	int32_t qs = 0, qe = read_i32(mTail.get());
-	while (qe > qs) {
-		hipLaunchKernelGGL(k_csr_closure_level, dim3(grid_blocks(qe - qs)), dim3(256), 0, mStream, qs, qe, mFirst.get(),
-		                   mHead.get(), mRes.get(), mS.get(), mQueue.get(), mTail.get());
+	CsrArgs args;
+	args.n = mN;
+	args.first = mFirst.get();
+	args.ends = mEnds.get();
+	args.pair = mPair.get();
+	args.e = mE.get();
+	args.rt = mRt.get();
+	args.h = mH.get();
+	args.mark = mS.get();
+	args.queue = mQueue.get();
+	args.list[0] = mList[0].get();
+	args.list[1] = mList[1].get();
+	args.starts = mLevelStarts.get();
+	args.ctl = mControl.get();
+	args.max_rounds = max_rounds;
+	args.stages = stages;
+	// Lanes per vertex: its arcs in one pass on average; twice that on small graphs, whose steps are
+	// short and take the more waves (19683 vertices, 7.8 arcs each: 16 lanes 1.8-2.1 ms, 8 lanes
+	// 2.0-2.2 ms; 1 M vertices: 8 lanes 24.8 ms, 16 lanes 24.7-27 ms).
+	const int64_t degree = mArcs / mN;
+	int group = degree <= 5 ? 4 : degree <= 12 ? 8 : degree <= 24 ? 16 : 32;
+	group = mN <= 32768 && group < 32 ? 2 * group : group;
+	// Workgroups: a barrier costs 1.4 us over 32 of them, 2.2 us over 64 and 3.8 us over 128, and
+	// wide steps want more (solve times: 512 vertices 0.27 ms on 1 and 0.33 ms on 2 workgroups; 5000: 2.2 ms
+	// on 1, 1.2 ms on 16; 64000: 3.3 / 2.9 / 3.0 / 3.5 ms on 16 / 32 / 64 / 96; 216000: 7.5 / 6.5 / 6.9 ms on
+	// 32 / 64 / 96; 1 M: 76 / 34 / 26 / 24.8 / 26 ms on 16 / 32 / 64 / 96 / 128).
+	int blocks = mN <= 1024 ? 1 : mN <= 65536 ? std::min(32, (mN + 255) / 256) : mN <= 524288 ? 64 : 96;
+	args.solo_limit = 128;  // entries of a step that workgroup 0 runs alone (0, 32 and 128 within 5 % each way)
+	void (*kernel)(CsrArgs) = group == 4    ? k_csr_solve<4>
+	                          : group == 8  ? k_csr_solve<8>
+	                          : group == 16 ? k_csr_solve<16>
+	                                        : k_csr_solve<32>;
+	for (;;) {
+		hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kCsrThreads), 0, mStream, args);
 		CGP_LAUNCH_CHECK();
-		++stats.cut_passes;
-		qs = qe;
-		qe = read_i32(mTail.get());
+		CGP_HIP(hipMemcpyAsync(mPinned.get(), mControl.get(), sizeof(CsrControl), hipMemcpyDeviceToHost, mStream));
+		CGP_HIP(hipStreamSynchronize(mStream));
+		if (blocks == 1 || mPinned[0].gate == kCsrGateOpen) {
+			break;
+		}
+		// the chip had no room for all workgroups at once: one workgroup needs no other
+		blocks = 1;
+		hipLaunchKernelGGL(k_csr_clear_words, dim3(1), dim3(64), 0, mStream, mControl.get());
+		CGP_LAUNCH_CHECK();
 	}
+	const CsrControl &ctl = *mPinned.get();
+	if (ctl.status == kCsrNotConverged) {
+		fail(CGP_ERR_NOT_CONVERGED, "max_rounds (" + std::to_string(max_rounds) + ") reached before convergence");
+	}
+	return ctl;
+}
+
+// The inflow of a vertex has to fit its int32 excess. Checked once per set of weights and t-links.
+void CsrSolver::check_headroom()
+{
+	if (mHeadroomChecked) {
+		return;
+	}
+	for (int v = 0; v < mN; ++v) {
+		const int64_t in = (v < (int)mIncoming.size() ? mIncoming[v] : 0) + mHostSource[v];
+		if (in > 0x7fffffffLL) {
+			fail(CGP_ERR_OVERFLOW, "vertex " + std::to_string(v) +
+			                           ": source capacity plus incoming capacities does not fit int32");
+		}
+	}
+	mHeadroomChecked = true;
 }
 
 int64_t CsrSolver::solve(const cgp_policy &policy, cgp_stats *stats_out, const TraceHook &trace)
@@ -598,13 +279,7 @@ int64_t CsrSolver::solve(const cgp_policy &policy, cgp_stats *stats_out, const T
 	if (policy.minimal_residual < 0.0f || !std::isfinite(policy.minimal_residual)) {
 		fail(CGP_ERR_INVALID, "minimal_residual must be finite and non-negative");
 	}
-	for (int v = 0; v < mN; ++v) {
-		const int64_t in = (v < (int)mIncoming.size() ? mIncoming[v] : 0) + mHostSource[v];
-		if (in > 0x7fffffffLL) {
-			fail(CGP_ERR_OVERFLOW, "vertex " + std::to_string(v) +
-			                           ": source capacity plus incoming capacities does not fit int32");
-		}
-	}
+	check_headroom();
 	cgp_stats stats;
 	std::memset(&stats, 0, sizeof(stats));
 	const auto t_start = std::chrono::steady_clock::now();
@@ -615,49 +290,55 @@ int64_t CsrSolver::solve(const cgp_policy &policy, cgp_stats *stats_out, const T
 	                        ? (int32_t)std::min<double>(std::floor((double)policy.minimal_residual), 2147483647.0)
 	                        : 0;
 
-	CGP_HIP(hipMemsetAsync(mFlow.get(), 0, mFlow.bytes(), mStream));
-	hipLaunchKernelGGL(k_csr_init_vertices, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mCs.get(), mCt.get(),
-	                   mE.get(), mRt.get());
-	if (mArcs > 0) {
-		hipLaunchKernelGGL(k_csr_copy, dim3(grid_blocks(mArcs)), dim3(256), 0, mStream, mArcs, mArcCap.get(), mRes.get());
-	}
+	hipLaunchKernelGGL(k_csr_init, dim3(grid_blocks(std::max<int64_t>(mN, mArcs))), dim3(256), 0, mStream, mN, mArcs,
+	                   mCs.get(), mCt.get(), mCap.get(), mE.get(), mRt.get(), mPair.get(), mControl.get(), threshold);
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipStreamSynchronize(mStream));
 	stats.init_ms = ms_since(t_start);
 	trace.emit(CGP_TRACE_STARTED, 0, 0, 0);
-
-	std::vector<int32_t> level_starts;
 	int iteration = 0;
-	for (;;) {
-		if (iteration >= max_rounds) {
-			fail(CGP_ERR_NOT_CONVERGED, "max_rounds (" + std::to_string(max_rounds) + ") reached before convergence");
-		}
-		trace.emit(CGP_TRACE_BEGIN_ITERATION, iteration, 0, 0);
-		auto t0 = std::chrono::steady_clock::now();
-		bfs(threshold, level_starts, stats);
-		stats.relabel_ms += ms_since(t0);
-		++stats.rounds;
-		trace.emit(CGP_TRACE_AFTER_RELABEL, iteration, 0, 0, level_starts.data(), (int)level_starts.size());
-		t0 = std::chrono::steady_clock::now();
-		const bool pushed = push_sweep(level_starts, stats);
-		stats.discharge_ms += ms_since(t0);
-		const bool done = !pushed && threshold == 0;
-		if (trace.fn) {
-			trace.emit(CGP_TRACE_AFTER_PUSH, iteration, done ? 1 : 0, read_flow());
-		}
-		++iteration;
-		if (!pushed) {
-			if (threshold > 0) {
-				threshold = 0;  // exact finish
-				continue;
-			}
-			break;
-		}
-	}
 	auto t0 = std::chrono::steady_clock::now();
-	source_closure(stats);
-	const int64_t flow = read_flow();
-	stats.cut_ms = ms_since(t0);
+	if (!trace.fn) {
+		const CsrControl &ctl = run_stages(kCsrRelabel | kCsrPush | kCsrLoop | kCsrClosure, max_rounds);
+		iteration = ctl.rounds;
+		stats.discharge_ms = ms_since(t0);
+	} else {
+		// one stage per launch, so that the hooks see the state in between
+		const auto next_launch = [&] {
+			hipLaunchKernelGGL(k_csr_clear_words, dim3(1), dim3(64), 0, mStream, mControl.get());
+			CGP_LAUNCH_CHECK();
+		};
+		std::vector<int32_t> level_starts;
+		for (bool done = false; !done; ++iteration) {
+			trace.emit(CGP_TRACE_BEGIN_ITERATION, iteration, 0, 0);
+			t0 = std::chrono::steady_clock::now();
+			next_launch();
+			const CsrControl &ctl = run_stages(kCsrRelabel, max_rounds);
+			done = ctl.status == kCsrDone;
+			level_starts.assign((size_t)std::max(ctl.levels, 1) + 1, 0);
+			CGP_HIP(hipMemcpyAsync(level_starts.data() + 1, mLevelStarts.get() + 1,
+			                       (level_starts.size() - 1) * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
+			CGP_HIP(hipStreamSynchronize(mStream));
+			stats.relabel_ms += ms_since(t0);
+			trace.emit(CGP_TRACE_AFTER_RELABEL, iteration, 0, 0, level_starts.data(), (int)level_starts.size());
+			t0 = std::chrono::steady_clock::now();
+			if (!done) {
+				next_launch();
+				run_stages(kCsrPush, max_rounds);
+			}
+			stats.discharge_ms += ms_since(t0);
+			trace.emit(CGP_TRACE_AFTER_PUSH, iteration, done ? 1 : 0, (int64_t)mPinned[0].flow);
+		}
+		t0 = std::chrono::steady_clock::now();
+		next_launch();
+		run_stages(kCsrClosure, max_rounds);
+		stats.cut_ms = ms_since(t0);
+	}
+	const CsrControl &ctl = *mPinned.get();
+	const int64_t flow = (int64_t)ctl.flow;
+	stats.rounds = ctl.rounds;
+	stats.bfs_passes = (int32_t)ctl.bfs_passes;
+	stats.discharge_phases = (int32_t)ctl.push_steps;
+	stats.cut_passes = (int32_t)ctl.cut_passes;
 	stats.flow = flow;
 	stats.total_ms = ms_since(t_start);
 	stats.voxels = mN;
@@ -674,11 +355,10 @@ void CsrSolver::sink_side(uint8_t *host_out, uint8_t mask, uint8_t background)
 	if (!mSolved) {
 		fail(CGP_ERR_STATE, "fill_segments before max_flow");
 	}
-	DeviceBuffer<uint8_t> tmp(mN);
-	hipLaunchKernelGGL(k_csr_masks, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mH.get(), mS.get(), tmp.get(), 0,
+	hipLaunchKernelGGL(k_csr_masks, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mH.get(), mS.get(), mMask.get(), 0,
 	                   mask, background);
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipMemcpyAsync(host_out, tmp.get(), mN, hipMemcpyDeviceToHost, mStream));
+	CGP_HIP(hipMemcpyAsync(host_out, mMask.get(), mN, hipMemcpyDeviceToHost, mStream));
 	CGP_HIP(hipStreamSynchronize(mStream));
 }
 
@@ -687,11 +367,10 @@ void CsrSolver::source_side(uint8_t *host_out)
 	if (!mSolved) {
 		fail(CGP_ERR_STATE, "source_set before max_flow");
 	}
-	DeviceBuffer<uint8_t> tmp(mN);
-	hipLaunchKernelGGL(k_csr_masks, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mH.get(), mS.get(), tmp.get(), 1,
+	hipLaunchKernelGGL(k_csr_masks, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mH.get(), mS.get(), mMask.get(), 1,
 	                   (uint8_t)1, (uint8_t)0);
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipMemcpyAsync(host_out, tmp.get(), mN, hipMemcpyDeviceToHost, mStream));
+	CGP_HIP(hipMemcpyAsync(host_out, mMask.get(), mN, hipMemcpyDeviceToHost, mStream));
 	CGP_HIP(hipStreamSynchronize(mStream));
 }
 

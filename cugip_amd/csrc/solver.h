@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "common.h"
+#include "csr_control.h"
 #include "grid_control.h"
 #include "grid_tile.h"
 
@@ -297,11 +298,8 @@ public:
 	                  std::vector<int32_t> &cs, std::vector<int32_t> &ct);
 
 private:
-	int bfs(int32_t threshold, std::vector<int32_t> &level_starts, cgp_stats &stats);
-	bool push_sweep(const std::vector<int32_t> &level_starts, cgp_stats &stats);
-	void source_closure(cgp_stats &stats);
-	int32_t read_i32(const int32_t *device_ptr);
-	int64_t read_flow();
+	void check_headroom();
+	const CsrControl &run_stages(int32_t stages, int32_t max_rounds);
 
 	hipStream_t mStream;
 	int mN = 0;
@@ -311,12 +309,16 @@ private:
 	std::vector<int32_t> mHostFirst;   // n + 1
 	std::vector<int64_t> mIncoming;    // sum of capacities into each vertex
 	std::vector<int32_t> mHostSource;  // source t-links (headroom check)
-	DeviceBuffer<int32_t> mFirst, mHead, mMate, mArcCap, mRes;
-	DeviceBuffer<int32_t> mCs, mCt, mE, mRt, mH, mQueue;
+	bool mHeadroomChecked = false;
+	DeviceBuffer<int32_t> mFirst;      // n + 1
+	DeviceBuffer<int2> mEnds;          // per arc: head, mate
+	DeviceBuffer<int2> mCap, mPair;    // per arc: capacity and residual, each with the mate's
+	DeviceBuffer<int32_t> mCs, mCt, mE, mRt, mH, mQueue, mList[2];
 	DeviceBuffer<int32_t> mS;          // S_min marks
-	DeviceBuffer<int32_t> mTail, mPushed, mStatus, mLevelStarts;
-	DeviceBuffer<unsigned long long> mFlow;
-	PinnedBuffer<int32_t> mPinned;
+	DeviceBuffer<uint8_t> mMask;       // read-backs
+	DeviceBuffer<int32_t> mLevelStarts;
+	DeviceBuffer<CsrControl> mControl;
+	PinnedBuffer<CsrControl> mPinned;
 };
 
 }  // namespace cgp

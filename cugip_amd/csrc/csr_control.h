@@ -12,15 +12,15 @@ enum CsrGate : int32_t { kCsrGateOpen = 1, kCsrGateClosed = 2 };
 // launches a relabel and the push steps that follow it one at a time.
 enum CsrStage : int32_t { kCsrRelabel = 1, kCsrPush = 2, kCsrLoop = 4, kCsrClosure = 8 };
 
-// Device control block; every phase (barrier interval) uses word phase % 3: low half the workgroups
-// that arrived, high half the entries appended to the list under construction. The word of the
-// next phase is cleared by workgroup 0 during a phase: it was last read two barriers before.
+// Device control block. Barrier i of a launch uses word i % 3 (csr_kernels.h has its fields); the word
+// of barrier i + 1 is cleared by workgroup 0 before it arrives at barrier i: it was last read at
+// barrier i - 2.
 struct CsrControl {
 	unsigned long long word[3];
 	unsigned long long flow;
-	int32_t active[2];   // length of the active list a relabel builds, by round parity
-	int32_t list_count;  // active vertices after the last relabel
-	int32_t levels;      // levels of the last relabel (queue ends in starts[1 .. levels])
+	int32_t held[2];     // vertices with excess that a relabel stored to memory, by round parity
+	int32_t list_count;  // vertices with excess after the last relabel
+	int32_t levels;      // levels of the last relabel (vertices up to each in starts[1 .. levels])
 	int32_t rounds, status, threshold;
 	int32_t arrived, gate;  // workgroups that started; whether the launch runs
 	int32_t solo[4];     // what workgroup 0 left after running short steps alone

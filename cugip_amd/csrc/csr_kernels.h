@@ -4,9 +4,12 @@
 // levels, push steps), each a short gather: what bounds it is the latency of a step, not bytes. So the
 // whole solve runs in one launch whose steps are separated by a barrier over few, large workgroups
 // (2-3 us at 64 workgroups of 1024 threads, against a launch and a host read of about 16 us per
-// level before), and a step whose list is short is run by workgroup 0 alone between workgroup barriers.
-// Measured (lattice-like graphs of 7.8 arcs a vertex): 1 M vertices 267 -> 25 ms, 19683 vertices
-// 22.3 -> 2.0 ms; a step of 1 M vertices' solve takes 9 us up to 4096 list entries and 22 us at 16-64 K.
+// level before), the lists of a step stay in LDS, and a step whose list is short is run by workgroup 0
+// alone between workgroup barriers.
+// Measured (lattice-like graphs of 7.8 arcs a vertex): 1 M vertices 347 -> 22 ms, 19683 vertices
+// 20 -> 2.1 ms. A push step of 1024-4096 vertices takes about 7 us there: vertex records 0.75, arcs
+// 1.2, neighbour labels 0.7, atomics 0.9, list 0.8, barrier 2 us; lists in memory instead of LDS cost
+// 1 us more a step (a chain of 20000 vertices, all short steps: 127 -> 65 ms).
 //
 // Between two relabels the push is synchronous push/relabel: every step takes each vertex that
 // holds excess, pushes along its admissible arcs (neighbour exactly one label lower) and raises
@@ -34,8 +37,9 @@ namespace cgp {
 
 constexpr int kCsrThreads = 1024;
 constexpr int kCsrWaves = kCsrThreads / 64;
-constexpr int kCsrStage = 4096;      // list entries a workgroup collects in LDS per step
-constexpr int kCsrMinSteps = 16;     // push steps after a relabel: twice its levels, at least this
+constexpr int kCsrStage = 4096;      // list entries a workgroup keeps in LDS
+constexpr int kCsrMinSteps = 16;     // push steps after a relabel: twice its levels, at least this many
+constexpr int kCsrMoreSteps = 128;   // and at most this many more than its levels
 constexpr long long kCsrGatherTicks = 25000000;  // wait for the launch's workgroups (100 MHz): 0.25 s
 
 struct CsrArgs {
@@ -44,118 +48,166 @@ struct CsrArgs {
 	const int2 *ends;
 	int2 *pair;
 	int32_t *e, *rt, *h, *mark;
-	int32_t *queue, *list[2];
-	int32_t *starts;  // n + 2: queue end after each level
+	int32_t *shared_list[2];  // n entries each
+	int32_t *held_list;       // n entries
+	int32_t *starts;          // n + 2: vertices labelled up to each level
 	CsrControl *ctl;
 	int32_t max_rounds;
 	int32_t stages;
-	int32_t solo_limit;  // list length that workgroup 0 runs alone
+	int32_t min_quota;   // entries a workgroup may keep of any step: what it takes in one pass
+	int32_t solo_limit;  // step length that workgroup 0 runs alone
 };
 
-// List entries of a workgroup, collected in LDS and stored by one reservation per step. (An atomic
-// per wave on one word serialises in the L2, about 12 ns each: over a level of 50000 vertices
-// that was most of the level's time.)
-struct CsrStageBuffer {
-	int32_t count, base;
-	int32_t entry[kCsrStage];
-};
-
+// Lists. A step takes a list of vertices and makes the next one. Each workgroup keeps the entries it
+// appends in LDS and takes them itself in the next step: no store, reservation and load of a list
+// between two steps. So that the work stays spread, it keeps no more than its quota (twice the mean
+// of the step); the entries beyond go to a list in memory that all workgroups share evenly.
 struct CsrShared {
-	CsrStageBuffer next, active;
-	unsigned long long seen;
+	int32_t entry[2][kCsrStage];  // by step parity: the list taken and the list made
+	int32_t count[3];             // entries appended, by step % 3 (the next one is zeroed a step ahead)
+	int32_t held[kCsrStage];      // vertices with excess that a relabel reached
+	int32_t held_count;
+	int32_t base;
 	int32_t gate;
+	unsigned long long seen;
 	long long red[kCsrWaves];
 };
 
-// What a workgroup knows of the running phase.
+// What a workgroup knows of the running step.
 struct CsrPhase {
-	unsigned index;
-	bool solo;  // no other workgroup takes part
+	unsigned index;            // barriers passed (the same in every workgroup)
+	unsigned step;             // steps this workgroup ran
+	bool solo;                 // no other workgroup takes part
+	int32_t local;             // entries in LDS
+	int32_t *from;             // entries in memory, and their number
+	int32_t shared;
+	int32_t total;             // entries of all workgroups
 };
+
+// A barrier's word: workgroups that arrived (8 bits), entries kept in LDS by them (22 bits), entries
+// reserved in the shared list (34 bits).
+constexpr int kCsrLocalShift = 8, kCsrSharedShift = 30;
+constexpr int kCsrMaxBlocks = 255;
+static_assert((long long)kCsrMaxBlocks * kCsrStage < 1ll << 22, "the entries in LDS fit their field");
 
 __device__ inline unsigned long long *phase_word(const CsrArgs &g, const CsrPhase &ph)
 {
 	return &g.ctl->word[ph.index % 3u];
 }
 
-// Where a step's entries go: a list under construction and the word that reserves places in it. A
-// workgroup that is the list's only writer needs no reservation (direct).
-struct CsrList {
-	int32_t *at;
-	unsigned long long *word;  // entries in the high half (the phase word)
-	int32_t *counter;          // or a plain count
-	bool direct;
-	__device__ int32_t reserve(int32_t entries) const
-	{
-		return word ? (int32_t)(atomicAdd(word, (unsigned long long)entries << 32) >> 32)
-		            : atomicAdd(counter, entries);
-	}
-};
-
-// Appends value where pred holds (all lanes of the wave take part). Entries beyond the LDS stage
-// are stored at once, with one reservation per wave.
-__device__ inline void stage_append(CsrStageBuffer &st, bool pred, int32_t value, const CsrList &list)
+// The shared list that the running step appends to.
+__device__ inline int32_t *shared_target(const CsrArgs &g, const CsrPhase &ph)
 {
-	const unsigned long long mask = __ballot(pred);
-	if (!mask) {
-		return;
-	}
+	return g.shared_list[(ph.index + 1u) & 1u];
+}
+
+// Reserves places in the shared list of the running step.
+__device__ inline int32_t reserve_shared(const CsrArgs &g, const CsrPhase &ph, int32_t entries)
+{
+	return (int32_t)(atomicAdd(phase_word(g, ph), (unsigned long long)entries << kCsrSharedShift) >> kCsrSharedShift);
+}
+
+// Places for the lanes' values where pred holds, in an LDS list with `count` entries so far: one
+// reservation for the wave and all kValues values of a lane. Returns the entries of the wave; place[i]
+// is that of value i.
+template <int kValues>
+__device__ inline int32_t wave_places(int32_t *count, const bool (&pred)[kValues], int32_t (&place)[kValues],
+                                      int32_t &base)
+{
 	const int lane = threadIdx.x & 63;
-	const int entries = (int)__popcll(mask);
-	int32_t base = 0;
+	int32_t entries = 0;
+#pragma unroll
+	for (int i = 0; i < kValues; ++i) {
+		const unsigned long long mask = __ballot(pred[i]);
+		place[i] = entries + (int)__popcll(mask & ((1ull << lane) - 1ull));
+		entries += (int)__popcll(mask);
+	}
+	if (entries == 0) {
+		return 0;
+	}
+	base = 0;
 	if (lane == 0) {
-		base = atomicAdd(&st.count, entries);
+		base = atomicAdd(count, entries);
 	}
 	base = __builtin_amdgcn_readfirstlane(base);
-	const int32_t p = base + (int)__popcll(mask & ((1ull << lane) - 1ull));
-	if (pred && p < kCsrStage) {
-		st.entry[p] = value;
+#pragma unroll
+	for (int i = 0; i < kValues; ++i) {
+		place[i] += base;
+	}
+	return entries;
+}
+
+// Appends values where pred holds to the list that the step makes (all lanes of the wave take part).
+// Entries beyond the LDS stage go to the shared list at once.
+template <int kValues>
+__device__ inline void append_next(const CsrArgs &g, CsrShared &sh, const CsrPhase &ph, const bool (&pred)[kValues],
+                                   const int32_t (&value)[kValues])
+{
+	int32_t place[kValues], base;
+	const int32_t entries = wave_places(&sh.count[(ph.step + 1u) % 3u], pred, place, base);
+	if (entries == 0) {
+		return;
+	}
+	int32_t *entry = sh.entry[(ph.step + 1u) & 1u];
+#pragma unroll
+	for (int i = 0; i < kValues; ++i) {
+		if (pred[i] && place[i] < kCsrStage) {
+			entry[place[i]] = value[i];
+		}
 	}
 	if (base + entries > kCsrStage) {  // (the same for the whole wave)
-		const int32_t from = base > kCsrStage ? base : kCsrStage;
-		int32_t place = from;
-		if (!list.direct) {
-			if (lane == 0) {
-				place = list.reserve(base + entries - from);
+		const int32_t beyond = base > kCsrStage ? base : kCsrStage;
+		int32_t at = beyond - kCsrStage;
+		if (!ph.solo) {
+			if ((threadIdx.x & 63) == 0) {
+				at = reserve_shared(g, ph, base + entries - beyond);
 			}
-			place = __builtin_amdgcn_readfirstlane(place);
+			at = __builtin_amdgcn_readfirstlane(at);
 		}
-		if (pred && p >= kCsrStage) {
-			list.at[place + (p - from)] = value;
+#pragma unroll
+		for (int i = 0; i < kValues; ++i) {
+			if (pred[i] && place[i] >= kCsrStage) {
+				shared_target(g, ph)[at + (place[i] - beyond)] = value[i];
+			}
 		}
 	}
 }
 
-// Stores the staged entries (after the last append) and empties the stage. Returns the entries of
-// this workgroup, those already stored among them.
-__device__ inline int32_t stage_flush(CsrStageBuffer &st, const CsrList &list)
+// The same for the vertices with excess that a relabel reaches.
+template <int kValues>
+__device__ inline void append_held(const CsrArgs &g, CsrShared &sh, int32_t *counter, const bool (&pred)[kValues],
+                                   const int32_t (&value)[kValues])
 {
-	__syncthreads();
-	const int32_t total = st.count;
-	const int32_t staged = total < kCsrStage ? total : kCsrStage;
-	if (total > 0) {  // (the same for the whole workgroup)
-		int32_t base = 0;
-		if (!list.direct) {
-			if (threadIdx.x == 0) {
-				st.base = list.reserve(staged);
-			}
-			__syncthreads();
-			base = st.base;
-		}
-		for (int i = threadIdx.x; i < staged; i += kCsrThreads) {
-			list.at[base + i] = st.entry[i];
-		}
-		__syncthreads();
-		if (threadIdx.x == 0) {
-			st.count = 0;
+	int32_t place[kValues], base;
+	const int32_t entries = wave_places(&sh.held_count, pred, place, base);
+	if (entries == 0) {
+		return;
+	}
+#pragma unroll
+	for (int i = 0; i < kValues; ++i) {
+		if (pred[i] && place[i] < kCsrStage) {
+			sh.held[place[i]] = value[i];
 		}
 	}
-	return total;
+	if (base + entries > kCsrStage) {
+		const int32_t beyond = base > kCsrStage ? base : kCsrStage;
+		int32_t at = 0;
+		if ((threadIdx.x & 63) == 0) {
+			at = atomicAdd(counter, base + entries - beyond);
+		}
+		at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+		for (int i = 0; i < kValues; ++i) {
+			if (pred[i] && place[i] >= kCsrStage) {
+				g.held_list[at + (place[i] - beyond)] = value[i];
+			}
+		}
+	}
 }
 
-// End of a phase over the grid. Returns the entries appended during it (by all workgroups). All stores
-// of the phase are visible to every workgroup afterwards.
-__device__ inline int32_t grid_phase_end(const CsrArgs &g, CsrShared &sh, CsrPhase &ph)
+// Barrier over the grid. All stores before it are visible to every workgroup afterwards. `local` is
+// what this workgroup keeps in LDS; ph.total and ph.shared get the sums over all.
+__device__ inline void grid_barrier(const CsrArgs &g, CsrShared &sh, CsrPhase &ph, int32_t local)
 {
 	// every wave's stores have reached the L2 before thread 0 writes the L2 back and arrives
 	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -164,21 +216,73 @@ __device__ inline int32_t grid_phase_end(const CsrArgs &g, CsrShared &sh, CsrPha
 	if (threadIdx.x == 0) {
 		unsigned long long *word = phase_word(g, ph);
 		if (blockIdx.x == 0) {
-			// the next phase's word (last read two barriers ago)
+			// the next barrier's word (last read two barriers ago)
 			__hip_atomic_store(&g.ctl->word[(ph.index + 1u) % 3u], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		}
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-		__hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		__hip_atomic_fetch_add(word, 1ull + ((unsigned long long)local << kCsrLocalShift), __ATOMIC_RELAXED,
+		                       __HIP_MEMORY_SCOPE_AGENT);
 		unsigned long long seen;
-		while ((uint32_t)(seen = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < gridDim.x) {
+		while (((seen = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 255ull) < gridDim.x) {
 			__builtin_amdgcn_s_sleep(1);
 		}
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 		sh.seen = seen;
 	}
 	__syncthreads();
+	const unsigned long long seen = sh.seen;
 	++ph.index;
-	return (int32_t)(sh.seen >> 32);
+	ph.shared = (int32_t)(seen >> kCsrSharedShift);
+	ph.total = ph.shared + (int32_t)((seen >> kCsrLocalShift) & ((1ull << (kCsrSharedShift - kCsrLocalShift)) - 1));
+}
+
+// Entries that a workgroup may keep of a step whose input has ph.total entries. A step of a list
+// short enough for workgroup 0 alone puts all of them into the shared list, where that one finds them.
+__device__ inline int32_t step_quota(const CsrArgs &g, const CsrPhase &ph)
+{
+	if (ph.total <= g.solo_limit) {
+		return 0;
+	}
+	const int32_t mean = ph.total / (int)gridDim.x, quota = mean + mean / 4;
+	return quota < g.min_quota ? g.min_quota : quota < kCsrStage ? quota : kCsrStage;
+}
+
+// End of a step: its list becomes the one to take.
+__device__ inline void step_end(const CsrArgs &g, CsrShared &sh, CsrPhase &ph)
+{
+	const unsigned next = ph.step + 1u;
+	if (threadIdx.x == 0) {
+		sh.count[(ph.step + 2u) % 3u] = 0;  // (the list before the one taken: nobody reads it any more)
+	}
+	__syncthreads();
+	const int32_t made = sh.count[next % 3u];
+	int32_t kept = made < kCsrStage ? made : kCsrStage;
+	if (ph.solo) {
+		ph.local = kept;
+		ph.shared = made - kept;
+		ph.total = made;
+		ph.from = shared_target(g, ph);
+		if (gridDim.x == 1) {
+			++ph.index;
+		}
+	} else {
+		const int32_t quota = step_quota(g, ph);
+		if (kept > quota) {  // (the same for the whole workgroup)
+			if (threadIdx.x == 0) {
+				sh.base = reserve_shared(g, ph, kept - quota);
+			}
+			__syncthreads();
+			int32_t *to = shared_target(g, ph) + sh.base;
+			for (int i = quota + (int)threadIdx.x; i < kept; i += kCsrThreads) {
+				to[i - quota] = sh.entry[next & 1u][i];
+			}
+			kept = quota;
+		}
+		ph.from = shared_target(g, ph);
+		grid_barrier(g, sh, ph, kept);
+		ph.local = kept;
+	}
+	ph.step = next;
 }
 
 // Before the first barrier: whether every workgroup of the launch is running. The barriers need that
@@ -209,195 +313,300 @@ __device__ inline bool all_running(const CsrArgs &g, CsrShared &sh)
 	return sh.gate == kCsrGateOpen;
 }
 
-// The list that a step appends to, starting at `at`.
-__device__ inline CsrList step_list(const CsrArgs &g, const CsrPhase &ph, int32_t *at)
+// The entries this workgroup takes: its own in LDS, then every gridDim.x-th run of kRun of the shared
+// list. Short runs: a CU handles one address of a gather a cycle, so even a few dozen entries are
+// worth spreading over the chip.
+template <int kRun>
+__device__ inline uint32_t own_entries(const CsrPhase &ph)
 {
-	return CsrList{at, ph.solo ? nullptr : phase_word(g, ph), nullptr, ph.solo};
+	const uint32_t blocks = ph.solo ? 1u : gridDim.x, block = ph.solo ? 0u : blockIdx.x;
+	const uint32_t runs = ((uint32_t)ph.shared + kRun - 1u) / kRun;
+	return (uint32_t)ph.local + (runs > block ? (runs - block + blocks - 1u) / blocks : 0u) * kRun;
 }
 
-// End of a step: the staged entries are stored to its list, and the number of entries that the step
-// appended is returned. A workgroup that runs alone only needs its own barriers.
-__device__ inline int32_t step_end(const CsrArgs &g, CsrShared &sh, CsrPhase &ph, const CsrList &list)
+// Entry i of them, or -1 (the end of the shared list's last run).
+template <int kRun>
+__device__ inline int32_t own_entry(const CsrShared &sh, const CsrPhase &ph, uint32_t i, uint32_t own)
 {
-	const int32_t own = stage_flush(sh.next, list);
-	if (ph.solo) {
-		__syncthreads();
-		return own;
+	if (i < (uint32_t)ph.local) {
+		return sh.entry[ph.step & 1u][i];
 	}
-	return grid_phase_end(g, sh, ph);
+	if (i >= own) {
+		return -1;
+	}
+	const uint32_t blocks = ph.solo ? 1u : gridDim.x, block = ph.solo ? 0u : blockIdx.x;
+	const uint32_t q = i - (uint32_t)ph.local;
+	const uint32_t at = (q / kRun * blocks + block) * kRun + q % kRun;
+	return at < (uint32_t)ph.shared ? ph.from[at] : -1;
 }
 
-// First list entry of this wave and the distance to its next ones: waves take kPer consecutive
-// entries, dealt out over the workgroups first, so that a short list spreads over all of them.
-template <int kPer>
-__device__ inline void wave_share(const CsrPhase &ph, int &begin, int &stride)
-{
-	const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-	const int blocks = ph.solo ? 1 : (int)gridDim.x;
-	const int block = ph.solo ? 0 : (int)blockIdx.x;
-	begin = (wave * blocks + block) * kPer;
-	stride = kCsrWaves * blocks * kPer;
-}
-
-// Start of a search: labels (or marks) of every vertex, the seeds into the queue. A relabel also
-// appends the vertices with excess that it reaches to the active list.
+// Start of a search: labels (or marks) of every vertex, the seeds into the list. A relabel also
+// collects the vertices with excess that it reaches.
 template <bool kClosure>
 __device__ inline void search_seed(const CsrArgs &g, CsrShared &sh, const CsrPhase &ph, int32_t threshold,
-                                   const CsrList &queue, const CsrList &active)
+                                   int32_t *held_counter)
 {
-	int begin, stride;
-	wave_share<64>(ph, begin, stride);
-	for (int64_t base = begin; base < g.n; base += stride) {
+	for (int64_t base = (int64_t)blockIdx.x * kCsrThreads + (threadIdx.x & ~63u); base < g.n;
+	     base += (int64_t)gridDim.x * kCsrThreads) {
 		const int64_t v = base + (threadIdx.x & 63);
-		bool seed = false, holds = false;
+		bool seed[1] = {false}, holds[1] = {false};
+		const int32_t value[1] = {(int32_t)v};
 		if (v < g.n) {
 			if (kClosure) {
-				seed = g.e[v] > 0;
-				g.mark[v] = seed ? 1 : 0;
+				seed[0] = g.e[v] > 0;
+				g.mark[v] = seed[0] ? 1 : 0;
 			} else {
-				seed = g.rt[v] > threshold;
-				holds = seed && g.e[v] > 0;
-				g.h[v] = seed ? 1 : kLabelInf;
+				seed[0] = g.rt[v] > threshold;
+				holds[0] = seed[0] && g.e[v] > 0;
+				g.h[v] = seed[0] ? 1 : kLabelInf;
 			}
 		}
-		stage_append(sh.next, seed, (int32_t)v, queue);
+		append_next(g, sh, ph, seed, value);
 		if (!kClosure) {
-			stage_append(sh.active, holds, (int32_t)v, active);
+			append_held(g, sh, held_counter, holds, value);
 		}
 	}
 }
 
-// One level: the unvisited neighbours u of the frontier queue[qs, qe) that can reach it (relabel:
-// residual u -> v > threshold) or that it reaches (closure: residual v -> u > 0).
-template <int kGroup, bool kClosure>
-__device__ inline void search_level(const CsrArgs &g, CsrShared &sh, const CsrPhase &ph, int qs, int qe, int32_t level,
-                                    int32_t threshold, const CsrList &queue, const CsrList &active)
+// One level: the unvisited neighbours u of the list's vertices v that can reach v (relabel: residual
+// u -> v > threshold) or that v reaches (closure: residual v -> u > 0).
+template <int kGroup, int kArcs, bool kClosure>
+__device__ inline void search_level(const CsrArgs &g, CsrShared &sh, const CsrPhase &ph, int32_t level,
+                                    int32_t threshold, int32_t *held_counter)
 {
 	constexpr int kPer = 64 / kGroup;
 	const int sub = threadIdx.x % kGroup, slot = (threadIdx.x & 63) / kGroup;
 	int32_t *visited = kClosure ? g.mark : g.h;
 	const int32_t fresh = kClosure ? 0 : kLabelInf;
-	int begin, stride;
-	wave_share<kPer>(ph, begin, stride);
-	const int count = qe - qs;
-	for (int64_t base = begin; base < count; base += stride) {
+	const uint32_t own = own_entries<kPer>(ph);
+	for (uint32_t base = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kPer; base < own;
+	     base += kCsrWaves * kPer) {
+		const int32_t v = own_entry<kPer>(sh, ph, base + slot, own);
 		uint32_t a = 0, end = 0;
-		if (base + slot < count) {
-			const int v = g.queue[qs + (int)base + slot];
+		if (v >= 0) {
 			a = (uint32_t)g.first[v] + sub;
 			end = (uint32_t)g.first[v + 1];
 		}
 		while (__any(a < end)) {
-			bool claimed = false, holds = false;
-			int u = 0;
-			if (a < end) {
-				u = g.ends[a].x;
-				const int2 p = g.pair[a];
-				if ((kClosure ? p.x > 0 : p.y > threshold) && visited[u] == fresh) {
-					claimed = atomicCAS(&visited[u], fresh, kClosure ? 1 : level + 1) == fresh;
-					holds = !kClosure && claimed && g.e[u] > 0;
+			int32_t u[kArcs], seen[kArcs], excess[kArcs];
+			bool open[kArcs], holds[kArcs];
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				u[i] = 0;
+				open[i] = false;
+				if (a + i * kGroup < end) {
+					u[i] = g.ends[a + i * kGroup].x;
+					const int2 p = g.pair[a + i * kGroup];
+					open[i] = kClosure ? p.x > 0 : p.y > threshold;
 				}
-				a += kGroup;
 			}
-			stage_append(sh.next, claimed, u, queue);
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				open[i] = open[i] && visited[u[i]] == fresh;
+			}
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				seen[i] = ~fresh;
+				excess[i] = 0;
+				if (open[i]) {
+					seen[i] = atomicCAS(&visited[u[i]], fresh, kClosure ? 1 : level + 1);
+					if (!kClosure) {
+						excess[i] = g.e[u[i]];
+					}
+				}
+			}
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				open[i] = seen[i] == fresh;
+				holds[i] = open[i] && excess[i] > 0;
+			}
+			append_next(g, sh, ph, open, u);
 			if (!kClosure) {
-				stage_append(sh.active, holds, u, active);
+				append_held(g, sh, held_counter, holds, u);
 			}
+			a += a < end ? (uint32_t)(kGroup * kArcs) : 0u;
 		}
 	}
 }
 
-// One synchronous push/relabel step over in[0, count); the vertices that hold excess after it (and
-// have a finite label) are appended to out, each once: a vertex of the list by itself when excess
-// is left, any other by the push that made its excess positive.
+// Values combined over the lanes of a group by DPP moves (no LDS round trips): lane exchanges inside
+// quads, then the mirrored half row and row; groups of 32 take one lane exchange more.
+template <int kGroup, typename Op>
+__device__ inline uint32_t group_all(uint32_t v, Op &&op)
+{
+	if constexpr (kGroup > 1) {
+		v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true));  // quad_perm 1 0 3 2
+	}
+	if constexpr (kGroup > 2) {
+		v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true));  // quad_perm 2 3 0 1
+	}
+	if constexpr (kGroup > 4) {
+		v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));  // row_half_mirror
+	}
+	if constexpr (kGroup > 8) {
+		v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));  // row_mirror
+	}
+	if constexpr (kGroup > 16) {
+		v = op(v, (uint32_t)__shfl_xor((int)v, 16, kGroup));
+	}
+	return v;
+}
+
+// Sum over the group's lanes before this one, held at `most` (every term and `most` below 2^31).
 template <int kGroup>
-__device__ inline void push_step(const CsrArgs &g, CsrShared &sh, const CsrPhase &ph, const int32_t *in, int count,
-                                 const CsrList &out, int32_t threshold, long long &sink)
+__device__ inline uint32_t group_sum_before(uint32_t v, uint32_t most, int sub)
+{
+	auto step = [&](uint32_t run, uint32_t o, int off) {
+		const uint32_t s = run + o;
+		return sub >= off ? (s < most ? s : most) : run;
+	};
+	uint32_t run = v;
+	if constexpr (kGroup > 1) {
+		run = step(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x111, 0xf, 0xf, true), 1);  // row_shr
+	}
+	if constexpr (kGroup > 2) {
+		run = step(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x112, 0xf, 0xf, true), 2);
+	}
+	if constexpr (kGroup > 4) {
+		run = step(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x114, 0xf, 0xf, true), 4);
+	}
+	if constexpr (kGroup > 8) {
+		run = step(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x118, 0xf, 0xf, true), 8);
+	}
+	if constexpr (kGroup > 16) {
+		run = step(run, (uint32_t)__shfl((int)run, 15, kGroup), 16);  // (the rows' sums so far are their own)
+	}
+	const uint32_t before = kGroup > 16 ? (uint32_t)__shfl_up((int)run, 1, kGroup)
+	                                    : (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x111, 0xf, 0xf, true);
+	return kGroup > 1 && sub > 0 ? before : 0u;
+}
+
+// One synchronous push/relabel step; the vertices that hold excess after it (and have a finite label)
+// are appended to the next list, each once: a vertex of the list by itself when excess is left, any
+// other by the push that made its excess positive.
+template <int kGroup, int kArcs>
+__device__ inline void push_step(const CsrArgs &g, CsrShared &sh, const CsrPhase &ph, int32_t threshold,
+                                 long long &sink)
 {
 	constexpr int kPer = 64 / kGroup;
 	const int sub = threadIdx.x % kGroup, slot = (threadIdx.x & 63) / kGroup;
-	int begin, stride;
-	wave_share<kPer>(ph, begin, stride);
-	for (int64_t base = begin; base < count; base += stride) {
-		int v = -1;
-		uint32_t at = 0, end = 0;       // next arcs of the group
-		int32_t x = 0, x0 = 0, hv = 0;  // excess left and at the start, label: the same in a group
-		if (base + slot < count) {
-			v = in[base + slot];
+	const uint32_t own = own_entries<kPer>(ph);
+	for (uint32_t base = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kPer; base < own;
+	     base += kCsrWaves * kPer) {
+		const int32_t v = own_entry<kPer>(sh, ph, base + slot, own);
+		uint32_t at = 0, end = 0;                // next arcs of the group
+		int32_t x = 0, hv = 0, rtv = 0;          // excess left, label, residual sink link
+		if (v >= 0) {
 			at = (uint32_t)g.first[v];
 			end = (uint32_t)g.first[v + 1];
-			x0 = x = g.e[v];
+			x = g.e[v];
 			hv = g.h[v];
-			const int32_t rtv = g.rt[v];
-			const int32_t fs = x < rtv ? x : rtv;
-			if (fs > 0) {
-				x -= fs;
-				if (sub == 0) {
-					g.rt[v] = rtv - fs;
-					sink += fs;
-				}
+			rtv = g.rt[v];
+		}
+		// one value per group, whatever is being added meanwhile
+		x = (int32_t)group_all<kGroup>((uint32_t)x, [](uint32_t p, uint32_t q) { return p < q ? p : q; });
+		const int32_t x0 = x;
+		int32_t left = x0, lowest = kLabelInf;
+		const int32_t fs = x < rtv ? x : rtv;
+		x -= fs;
+		bool go = x > 0 && at < end;
+		if (fs > 0 && sub == 0) {
+			g.rt[v] = rtv - fs;
+			sink += fs;
+			if (!go) {
+				left = atomicSub(&g.e[v], fs) - fs;
 			}
 		}
-		int32_t lowest = kLabelInf;
-		while (__any(x > 0 && at < end)) {
-			const bool go = x > 0 && at < end;
-			const uint32_t a = at + sub;
-			const bool own = go && a < end;
-			int2 ends = make_int2(0, 0), p = make_int2(0, 0);
-			int32_t l = kLabelInf;
-			if (own) {
-				ends = g.ends[a];
-				p = g.pair[a];
-				l = g.h[ends.x];
-			}
-			const bool open = own && p.x > threshold;
-			const bool admissible = open && l == hv - 1;
-			// the group's admissible residuals in arc order share the excess: running sums held at x
-			const uint32_t cap = admissible ? (uint32_t)(p.x < x ? p.x : x) : 0u;
-			uint32_t run = cap;
+		bool woken[kArcs + 1];
+		int32_t value[kArcs + 1];
 #pragma unroll
-			for (int off = 1; off < kGroup; off <<= 1) {
-				const uint32_t o = (uint32_t)__shfl_up((int)run, off, kGroup);
-				const uint32_t s = run + o;
-				run = sub >= off ? (s < (uint32_t)x ? s : (uint32_t)x) : run;
+		for (int i = 0; i <= kArcs; ++i) {
+			woken[i] = false;
+			value[i] = 0;
+		}
+		for (bool more = __any(go); more;) {
+			int2 ends[kArcs], p[kArcs];
+			int32_t l[kArcs], old[kArcs];
+			uint32_t cap[kArcs];
+			bool arc[kArcs];
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				const uint32_t a = at + sub + i * kGroup;
+				arc[i] = go && a < end;
+				ends[i] = p[i] = make_int2(0, 0);
+				if (arc[i]) {
+					ends[i] = g.ends[a];
+					p[i] = g.pair[a];
+				}
 			}
-			uint32_t before = (uint32_t)__shfl_up((int)run, 1, kGroup);
-			before = sub == 0 ? 0u : before;
-			const uint32_t room = (uint32_t)x - before;
-			const int32_t f = (int32_t)(cap < room ? cap : room);
-			const int32_t total = __shfl((int)run, kGroup - 1, kGroup);
-			bool woken = false;
-			if (f > 0) {
-				g.pair[a] = make_int2(p.x - f, p.y + f);
-				g.pair[ends.y] = make_int2(p.y + f, p.x - f);
-				woken = atomicAdd(&g.e[ends.x], f) == 0;
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				l[i] = arc[i] ? g.h[ends[i].x] : kLabelInf;
 			}
-			stage_append(sh.next, woken, ends.x, out);
-			if (own && ((open && !admissible) || (l > hv && p.y > threshold))) {
-				lowest = l < lowest ? l : lowest;
+			// the group's admissible residuals share the excess: the lanes' sums, held at x, then their
+			// running sums over the group
+			uint32_t mine = 0;
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				const bool open = arc[i] && p[i].x > threshold;
+				const bool admissible = open && l[i] == hv - 1;
+				cap[i] = admissible ? (uint32_t)(p[i].x < x ? p[i].x : x) : 0u;
+				mine = mine + cap[i] < (uint32_t)x ? mine + cap[i] : (uint32_t)x;
+				if (arc[i] && ((open && !admissible) || (l[i] > hv && p[i].y > threshold))) {
+					lowest = l[i] < lowest ? l[i] : lowest;
+				}
+			}
+			const uint32_t most = (uint32_t)x;
+			const int32_t total = (int32_t)group_all<kGroup>(
+			    mine, [&](uint32_t p, uint32_t q) { return p + q < most ? p + q : most; });
+			const uint32_t before = group_sum_before<kGroup>(mine, most, sub);
+			uint32_t room = (uint32_t)x - before;
+#pragma unroll
+			for (int i = 0; i < kArcs; ++i) {
+				const int32_t f = (int32_t)(cap[i] < room ? cap[i] : room);
+				room -= (uint32_t)f;
+				old[i] = 1;
+				if (f > 0) {
+					g.pair[at + sub + i * kGroup] = make_int2(p[i].x - f, p[i].y + f);
+					g.pair[ends[i].y] = make_int2(p[i].y + f, p[i].x - f);
+					old[i] = atomicAdd(&g.e[ends[i].x], f);
+				}
 			}
 			x -= total;
-			at += go ? (uint32_t)kGroup : 0u;
-		}
+			at += go ? (uint32_t)(kGroup * kArcs) : 0u;
+			const bool again = x > 0 && at < end;
+			// the last arcs of v: what it sent leaves its excess (together with the receivers' adds)
+			if (go && !again && sub == 0 && x < x0) {
+				left = atomicSub(&g.e[v], x0 - x) - (x0 - x);
+			}
+			go = again;
+			more = __any(go);
 #pragma unroll
-		for (int off = kGroup / 2; off > 0; off >>= 1) {
-			const int32_t o = __shfl_xor(lowest, off, kGroup);
-			lowest = o < lowest ? o : lowest;
-		}
-		bool again = false;
-		if (v >= 0 && sub == 0 && x0 > 0) {
-			const int32_t sent = x0 - x;
-			const int32_t left = sent > 0 ? atomicSub(&g.e[v], sent) - sent : x0;
-			int32_t label = hv;
-			if (x > 0) {
-				const int32_t raised = lowest < kLabelInf ? lowest + 1 : kLabelInf;
-				if (raised > hv) {
-					g.h[v] = label = raised;
+			for (int i = 0; i < kArcs; ++i) {
+				value[i] = ends[i].x;
+				woken[i] = old[i] == 0;
+			}
+			if (more) {
+				append_next(g, sh, ph, woken, value);
+#pragma unroll
+				for (int i = 0; i < kArcs; ++i) {
+					woken[i] = false;
 				}
 			}
-			again = left > 0 && label < kLabelInf;
 		}
-		stage_append(sh.next, again, v, out);
+		lowest = (int32_t)group_all<kGroup>((uint32_t)lowest, [](uint32_t p, uint32_t q) { return p < q ? p : q; });
+		int32_t label = hv;
+		const bool lead = v >= 0 && sub == 0 && x0 > 0;
+		if (lead && x > 0) {
+			const int32_t raised = lowest < kLabelInf ? lowest + 1 : kLabelInf;
+			if (raised > hv) {
+				g.h[v] = label = raised;
+			}
+		}
+		// the vertices woken by the last arcs and v itself, with one reservation
+		woken[kArcs] = lead && left > 0 && label < kLabelInf;
+		value[kArcs] = v;
+		append_next(g, sh, ph, woken, value);
 	}
 }
 
@@ -407,67 +616,108 @@ __device__ inline int32_t told(const int32_t *word)
 	return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A breadth-first search from its seeds. Returns the number of levels; a relabel's queue
-// ends go to starts[1 ..], its active list to list[0] with its length in active_count.
-template <int kGroup, bool kClosure>
-__device__ inline int search(const CsrArgs &g, CsrShared &sh, CsrPhase &ph, int32_t threshold, int parity,
-                             int32_t &active_count)
+// Runs steps i, i + 1, ... below limit while the list has entries; returns the next i. step(i) runs
+// one, done(i) is called by workgroup 0 after each.
+template <typename Step, typename Done>
+__device__ inline int run_steps(const CsrArgs &g, CsrShared &sh, CsrPhase &ph, int i, int limit, Step &&step,
+                                Done &&done)
+{
+	const bool alone = gridDim.x == 1;
+	while (i < limit && ph.total > 0) {
+		if (alone || ph.total > g.solo_limit || ph.shared < ph.total) {
+			step(i);
+			step_end(g, sh, ph);
+			++i;
+			if (blockIdx.x == 0) {
+				done(i);
+			}
+			continue;
+		}
+		// the whole list is short and in the shared list: workgroup 0 takes it and runs the steps that
+		// follow while they stay short; the others wait for it at the barrier
+		if (blockIdx.x == 0) {
+			const int32_t entries = ph.shared;
+			if ((int)threadIdx.x < entries) {  // solo_limit <= kCsrThreads
+				sh.entry[ph.step & 1u][threadIdx.x] = ph.from[threadIdx.x];
+			}
+			ph.local = entries;
+			ph.shared = 0;
+			ph.solo = true;
+			__syncthreads();
+			do {
+				step(i);
+				step_end(g, sh, ph);
+				__syncthreads();
+				++i;
+				done(i);
+			} while (i < limit && ph.total > 0 && ph.total <= 4 * g.solo_limit);
+			ph.solo = false;
+			// back into the shared list, after what did not fit the LDS stage
+			int32_t *to = shared_target(g, ph) + ph.shared;
+			for (int k = threadIdx.x; k < ph.local; k += kCsrThreads) {
+				to[k] = sh.entry[ph.step & 1u][k];
+			}
+			if (threadIdx.x == 0) {
+				g.ctl->solo[0] = i;
+				g.ctl->solo[1] = ph.total;
+			}
+		}
+		ph.from = shared_target(g, ph);
+		grid_barrier(g, sh, ph, 0);
+		i = told(&g.ctl->solo[0]);
+		ph.total = ph.shared = told(&g.ctl->solo[1]);
+		ph.local = 0;
+	}
+	return i;
+}
+
+// A breadth-first search from its seeds. Returns the number of levels; the vertices up to each level of
+// a relabel go to starts[1 ..], and its list of vertices with excess is the next step's input.
+template <int kGroup, int kArcs, bool kClosure>
+__device__ inline int search(const CsrArgs &g, CsrShared &sh, CsrPhase &ph, int32_t threshold, int parity)
 {
 	const bool alone = gridDim.x == 1;
 	const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
-	int32_t *counter = &g.ctl->active[parity];
-	const CsrList active{g.list[0], nullptr, counter, alone};
-	CsrList queue = step_list(g, ph, g.queue);
-	search_seed<kClosure>(g, sh, ph, threshold, queue, active);
-	int32_t got = step_end(g, sh, ph, queue);
-	int level = 1, qs = 0, qe = got;
+	int32_t *counter = &g.ctl->held[parity];
+	// the last list is dropped
+	ph.local = ph.shared = 0;
+	ph.total = g.n;
+	search_seed<kClosure>(g, sh, ph, threshold, counter);
+	step_end(g, sh, ph);
+	int32_t labelled = ph.total;
 	if (!kClosure && writer) {
-		g.starts[1] = qe;
+		g.starts[1] = labelled;
 		// the other round's count: every workgroup has read it before the barrier just passed
-		__hip_atomic_store(&g.ctl->active[parity ^ 1], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		__hip_atomic_store(&g.ctl->held[parity ^ 1], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	}
-	while (got > 0) {
-		const bool handover = !alone && got <= g.solo_limit;
-		if (handover) {
-			// workgroup 0 runs the levels that follow while they stay short; the others wait for it
-			if (blockIdx.x == 0) {
-				ph.solo = true;
-			}
-		}
-		if (!handover || blockIdx.x == 0) {
-			do {
-				queue = step_list(g, ph, g.queue + qe);
-				search_level<kGroup, kClosure>(g, sh, ph, qs, qe, level, threshold, queue, active);
-				got = step_end(g, sh, ph, queue);
-				qs = qe;
-				qe += got;
-				++level;
-				if (!kClosure && writer && got > 0) {
-					g.starts[level] = qe;
-				}
-			} while (handover && got > 0 && got <= 4 * g.solo_limit);
-		}
-		if (handover) {
-			ph.solo = false;
-			if (writer) {
-				g.ctl->solo[0] = level;
-				g.ctl->solo[1] = qs;
-				g.ctl->solo[2] = qe;
-			}
-			grid_phase_end(g, sh, ph);
-			level = told(&g.ctl->solo[0]);
-			qs = told(&g.ctl->solo[1]);
-			qe = told(&g.ctl->solo[2]);
-			got = qe - qs;
-		}
-	}
+	const int level = run_steps(
+	    g, sh, ph, 1, 0x7fffffff,
+	    [&](int at) { search_level<kGroup, kArcs, kClosure>(g, sh, ph, at, threshold, counter); },
+	    [&](int at) {
+		    if (!kClosure && threadIdx.x == 0 && ph.total > 0) {
+			    g.starts[at] = labelled += ph.total;
+		    }
+	    });
 	if (!kClosure) {
-		active_count = stage_flush(sh.active, active);
+		__syncthreads();
+		const int32_t held = sh.held_count;
+		ph.local = held < kCsrStage ? held : kCsrStage;
+		for (int k = threadIdx.x; k < ph.local; k += kCsrThreads) {
+			sh.entry[ph.step & 1u][k] = sh.held[k];
+		}
 		if (alone) {
 			__syncthreads();
+			ph.total = held;
+			ph.shared = held - ph.local;
 		} else {
-			grid_phase_end(g, sh, ph);
-			active_count = told(counter);
+			const int32_t local = ph.local;
+			grid_barrier(g, sh, ph, local);
+			ph.shared = told(counter);
+			ph.total += ph.shared;
+		}
+		ph.from = g.held_list;
+		if (threadIdx.x == 0) {
+			sh.held_count = 0;
 		}
 	}
 	return level - 1;
@@ -475,13 +725,15 @@ __device__ inline int search(const CsrArgs &g, CsrShared &sh, CsrPhase &ph, int3
 
 // The stages of g.stages. The control block's barrier words, arrival count and gate must be zero, the
 // rest as the last launch of the solve left it.
-template <int kGroup>
+template <int kGroup, int kArcs>
 __global__ __launch_bounds__(kCsrThreads) void k_csr_solve(CsrArgs g)
 {
 	__shared__ CsrShared sh;
+	if (threadIdx.x < 3) {
+		sh.count[threadIdx.x] = 0;
+	}
 	if (threadIdx.x == 0) {
-		sh.next.count = 0;
-		sh.active.count = 0;
+		sh.held_count = 0;
 	}
 	__syncthreads();
 	const bool alone = gridDim.x == 1;
@@ -489,8 +741,13 @@ __global__ __launch_bounds__(kCsrThreads) void k_csr_solve(CsrArgs g)
 		return;
 	}
 	const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
-	CsrPhase ph{0u, alone};
-	int32_t threshold = g.ctl->threshold, rounds = g.ctl->rounds, count = g.ctl->list_count, levels = g.ctl->levels;
+	CsrPhase ph;
+	ph.index = ph.step = 0;
+	ph.solo = alone;
+	ph.local = 0;
+	ph.from = g.held_list;
+	ph.total = ph.shared = g.ctl->list_count;  // the list that a relabel of its own launch left
+	int32_t threshold = g.ctl->threshold, rounds = g.ctl->rounds, levels = g.ctl->levels;
 	int32_t status = g.ctl->status;
 	long long sink = 0, passes = 0, steps = 0, cut_passes = 0;
 	for (;;) {
@@ -499,10 +756,10 @@ __global__ __launch_bounds__(kCsrThreads) void k_csr_solve(CsrArgs g)
 				status = kCsrNotConverged;
 				break;
 			}
-			levels = search<kGroup, false>(g, sh, ph, threshold, rounds & 1, count);
+			levels = search<kGroup, kArcs, false>(g, sh, ph, threshold, rounds & 1);
 			++rounds;
 			passes += levels;
-			if (count == 0) {
+			if (ph.total == 0) {
 				if (threshold == 0) {
 					status = kCsrDone;
 					break;
@@ -511,41 +768,28 @@ __global__ __launch_bounds__(kCsrThreads) void k_csr_solve(CsrArgs g)
 			}
 		}
 		if (g.stages & kCsrPush) {
-			const int limit = levels > kCsrMinSteps / 2 ? 2 * levels : kCsrMinSteps;
-			int i = 0;
-			while (i < limit && count > 0) {
-				const bool handover = !alone && count <= g.solo_limit;
-				if (handover && blockIdx.x == 0) {
-					ph.solo = true;
-				}
-				if (!handover || blockIdx.x == 0) {
-					do {
-						const CsrList out = step_list(g, ph, g.list[(i & 1) ^ 1]);
-						push_step<kGroup>(g, sh, ph, g.list[i & 1], count, out, threshold, sink);
-						count = step_end(g, sh, ph, out);
-						++i;
-					} while (handover && i < limit && count > 0 && count <= 4 * g.solo_limit);
-				}
-				if (handover) {
-					ph.solo = false;
-					if (writer) {
-						g.ctl->solo[0] = i;
-						g.ctl->solo[1] = count;
-					}
-					grid_phase_end(g, sh, ph);
-					i = told(&g.ctl->solo[0]);
-					count = told(&g.ctl->solo[1]);
-				}
-			}
-			steps += i;
+			const int limit = levels > kCsrMinSteps / 2 ? levels + (levels < kCsrMoreSteps ? levels : kCsrMoreSteps)
+			                                            : kCsrMinSteps;
+			steps += run_steps(
+			    g, sh, ph, 0, limit, [&](int) { push_step<kGroup, kArcs>(g, sh, ph, threshold, sink); }, [](int) {});
 		}
 		if (!(g.stages & kCsrLoop)) {
 			break;
 		}
 	}
+	if (g.stages == kCsrRelabel) {
+		// for the push steps of the next launch: the list goes to memory
+		__shared__ int32_t at;
+		if (threadIdx.x == 0) {
+			at = ph.local ? atomicAdd(&g.ctl->held[(rounds & 1) ^ 1], ph.local) : 0;
+		}
+		__syncthreads();
+		for (int k = threadIdx.x; k < ph.local; k += kCsrThreads) {
+			g.held_list[at + k] = sh.entry[ph.step & 1u][k];
+		}
+	}
 	if ((g.stages & kCsrClosure) && status == kCsrDone) {
-		int32_t unused;
-		cut_passes = search<kGroup, true>(g, sh, ph, 0, 0, unused);
+		cut_passes = search<kGroup, kArcs, true>(g, sh, ph, 0, 0);
 	}
 	__syncthreads();
 	const long long total = block_sum_i64<kCsrThreads>(sink, sh.red);
@@ -555,12 +799,21 @@ __global__ __launch_bounds__(kCsrThreads) void k_csr_solve(CsrArgs g)
 	if (writer) {
 		g.ctl->threshold = threshold;
 		g.ctl->rounds = rounds;
-		g.ctl->list_count = count;
+		g.ctl->list_count = ph.total;
 		g.ctl->levels = levels;
 		g.ctl->status = status;
 		g.ctl->bfs_passes += passes;
 		g.ctl->push_steps += steps;
 		g.ctl->cut_passes = cut_passes;
+	}
+}
+
+// Every arc's capacity next to its mate's.
+__global__ __launch_bounds__(256) void k_csr_pair_caps(int64_t arcs, const int2 *__restrict__ ends,
+                                                       const int32_t *__restrict__ own, int2 *__restrict__ cap)
+{
+	for (int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; a < arcs; a += (int64_t)gridDim.x * blockDim.x) {
+		cap[a] = make_int2(own[a], own[ends[a].y]);
 	}
 }
 

@@ -15,6 +15,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <memory>
 
 #include "common.h"
 #include "csr_kernels.h"
@@ -66,7 +67,7 @@ void CsrSolver::set_vertex_count(int n)
 	mE.allocate(n);
 	mRt.allocate(n);
 	mH.allocate(n);
-	mQueue.allocate(n);
+	mHeld.allocate(n);
 	mList[0].allocate(n);
 	mList[1].allocate(n);
 	mS.allocate(n);
@@ -116,7 +117,8 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 	}
 	const int64_t arcs = first[mN];
 	std::vector<int32_t> pos(first.begin(), first.end() - 1);
-	std::vector<int2> ends(arcs), cap(arcs);  // {head, mate}, {capacity, the mate's capacity}
+	const std::unique_ptr<int2[]> ends(new int2[arcs]);  // {head, mate}; every entry is written below
+	const std::unique_ptr<int32_t[]> cap(new int32_t[arcs]);
 	std::vector<int64_t> incoming(mN, 0);
 	for (int i = 0; i < m; ++i) {
 		const int a = (int)edges[i].first, b = (int)edges[i].second;
@@ -125,9 +127,9 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 		}
 		const int ia = pos[a]++, ib = pos[b]++;
 		ends[ia] = make_int2(b, ib);
-		cap[ia] = make_int2(fwd[i], bwd[i]);
+		cap[ia] = fwd[i];
 		ends[ib] = make_int2(a, ia);
-		cap[ib] = make_int2(bwd[i], fwd[i]);
+		cap[ib] = bwd[i];
 		incoming[b] += fwd[i];
 		incoming[a] += bwd[i];
 	}
@@ -142,8 +144,13 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 		mEnds.allocate(arcs);
 		mCap.allocate(arcs);
 		mPair.allocate(arcs);
-		CGP_HIP(hipMemcpyAsync(mEnds.get(), ends.data(), arcs * sizeof(int2), hipMemcpyHostToDevice, mStream));
-		CGP_HIP(hipMemcpyAsync(mCap.get(), cap.data(), arcs * sizeof(int2), hipMemcpyHostToDevice, mStream));
+		// the capacities travel through the residuals' memory, which the solve writes first
+		int32_t *own = reinterpret_cast<int32_t *>(mPair.get());
+		CGP_HIP(hipMemcpyAsync(mEnds.get(), ends.get(), arcs * sizeof(int2), hipMemcpyHostToDevice, mStream));
+		CGP_HIP(hipMemcpyAsync(own, cap.get(), arcs * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
+		hipLaunchKernelGGL(k_csr_pair_caps, dim3(grid_blocks(arcs)), dim3(256), 0, mStream, arcs, mEnds.get(), own,
+		                   mCap.get());
+		CGP_LAUNCH_CHECK();
 	}
 	CGP_HIP(hipStreamSynchronize(mStream));
 }
@@ -212,29 +219,29 @@ const CsrControl &CsrSolver::run_stages(int32_t stages, int32_t max_rounds)
 	args.rt = mRt.get();
 	args.h = mH.get();
 	args.mark = mS.get();
-	args.queue = mQueue.get();
-	args.list[0] = mList[0].get();
-	args.list[1] = mList[1].get();
+	args.shared_list[0] = mList[0].get();
+	args.shared_list[1] = mList[1].get();
+	args.held_list = mHeld.get();
 	args.starts = mLevelStarts.get();
 	args.ctl = mControl.get();
 	args.max_rounds = max_rounds;
 	args.stages = stages;
-	// Lanes per vertex: its arcs in one pass on average; twice that on small graphs, whose steps are
-	// short and take the more waves (19683 vertices, 7.8 arcs each: 16 lanes 1.8-2.1 ms, 8 lanes
-	// 2.0-2.2 ms; 1 M vertices: 8 lanes 24.8 ms, 16 lanes 24.7-27 ms).
+	// Lanes per vertex (two arcs each): the arcs of most vertices in one pass, since a second one costs a
+	// step another round of loads (1 M vertices of 7.8 arcs: 8 lanes of 2 arcs 22.2 ms, 16 of 1
+	// 26.7 ms, 4 of 2 26.8 ms, 8 of 1 28 ms; 19683 vertices: 2.2, 2.0, 2.7 and 2.3 ms).
 	const int64_t degree = mArcs / mN;
-	int group = degree <= 5 ? 4 : degree <= 12 ? 8 : degree <= 24 ? 16 : 32;
-	group = mN <= 32768 && group < 32 ? 2 * group : group;
+	const int group = degree <= 5 ? 4 : degree <= 12 ? 8 : degree <= 24 ? 16 : 32;
+	void (*kernel)(CsrArgs) = group == 4    ? k_csr_solve<4, 2>
+	                          : group == 8  ? k_csr_solve<8, 2>
+	                          : group == 16 ? k_csr_solve<16, 2>
+	                                        : k_csr_solve<32, 2>;
 	// Workgroups: a barrier costs 1.4 us over 32 of them, 2.2 us over 64 and 3.8 us over 128, and
-	// wide steps want more (solve times: 512 vertices 0.27 ms on 1 and 0.33 ms on 2 workgroups; 5000: 2.2 ms
-	// on 1, 1.2 ms on 16; 64000: 3.3 / 2.9 / 3.0 / 3.5 ms on 16 / 32 / 64 / 96; 216000: 7.5 / 6.5 / 6.9 ms on
-	// 32 / 64 / 96; 1 M: 76 / 34 / 26 / 24.8 / 26 ms on 16 / 32 / 64 / 96 / 128).
-	int blocks = mN <= 1024 ? 1 : mN <= 65536 ? std::min(32, (mN + 255) / 256) : mN <= 524288 ? 64 : 96;
-	args.solo_limit = 128;  // entries of a step that workgroup 0 runs alone (0, 32 and 128 within 5 % each way)
-	void (*kernel)(CsrArgs) = group == 4    ? k_csr_solve<4>
-	                          : group == 8  ? k_csr_solve<8>
-	                          : group == 16 ? k_csr_solve<16>
-	                                        : k_csr_solve<32>;
+	// wide steps want more (512 vertices: 0.21 ms on 1 workgroup, 0.33 ms on 2; 5000: 1.2 / 1.1 ms on
+	// 8 / 16; 19683: 2.6 / 2.3 / 2.2 / 2.4 ms on 8 / 16 / 32 / 64; 64000: 3.1 / 2.4 / 2.5 / 2.8 ms on 16 / 32 / 64 / 96;
+	// 216000: 6.7 / 6.2 / 6.5 ms on 32 / 64 / 96; 1 M: 23.1 / 22.2 / 23.6 ms on 64 / 96 / 128).
+	int blocks = mN <= 1024 ? 1 : mN <= 131072 ? std::min(32, (mN + 255) / 256) : mN <= 524288 ? 64 : 96;
+	args.min_quota = kCsrThreads / group;  // (0, 8 and 32 for 8 lanes: 2 to 8 % slower)
+	args.solo_limit = 128;
 	for (;;) {
 		hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kCsrThreads), 0, mStream, args);
 		CGP_LAUNCH_CHECK();

@@ -59,7 +59,7 @@ private:
 	DeviceBuffer<uint16_t> mG[2];                 // pre-activation gradients (ping-pong)
 	DeviceBuffer<float> mLogit;
 	DeviceBuffer<uint8_t> mVolume, mSide;
-	DeviceBuffer<double> mScalars;                // loss and head-bias gradient accumulators
+	DeviceBuffer<double2> mScalars;               // loss and head-bias gradient: the sum, then per-block sums
 	int mStep = 0;
 	bool mPackDirty = true;
 };

@@ -115,25 +115,6 @@ __global__ __launch_bounds__(256) void k_cnn_input(int64_t n, const uint8_t *__r
 	}
 }
 
-// Stage the input brick (channel-last, CIN channels) with its halo; zero outside the volume.
-template <int CIN>
-__device__ inline void stage_brick(uint16_t *lds, const uint16_t *__restrict__ in, int nx, int ny, int nz, int bx,
-                                   int by, int bz)
-{
-	constexpr int kParts = CIN / 4;  // 8-byte units per voxel
-	for (int e = threadIdx.x; e < HV * kParts; e += blockDim.x) {
-		const int hv = e / kParts, part = e % kParts;
-		const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-		const int x = bx + hx - 1, y = by + hy - 1, z = bz + hz - 1;
-		uint2 val = make_uint2(0u, 0u);
-		if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) {
-			const int64_t v = ((int64_t)z * ny + y) * nx + x;
-			val = *reinterpret_cast<const uint2 *>(in + v * CIN + part * 4);
-		}
-		*reinterpret_cast<uint2 *>(lds + hv * CIN + part * 4) = val;
-	}
-}
-
 // Stage the input brick with its halo as one plane per group of 4 channels (8 bytes a voxel), so
 // that the 16 lanes of an MFMA B fragment, which read one channel group of 16 consecutive voxels,
 // read 128 contiguous bytes (channel-last, their 8-byte reads would stride 32 bytes and collide in
@@ -418,124 +399,257 @@ __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, cons
 }
 
 // Weight gradient of one layer: dW[t][ci][co] = sum_v in[v + off(t)][ci] * g[v][co] and
-// db[co] = sum_v g[v][co], as D = A x B over chunks of 16 voxels: A = in^T (ci x voxel, from the
-// input brick), B = g (voxel x co). Wave w owns taps w, w + 4, ...; a workgroup walks bricks with a
-// grid stride and writes its partial sums (27*CIN*16 weights, then 16 biases) to partial[block].
+// db[co] = sum_v g[v][co], as D = A x B over the voxels: A = in^T (ci x voxel, from the input brick),
+// B = g (voxel x co), two rows of 16 voxels per v_mfma_f32_16x16x32_bf16 (the k index of lane group grp is
+// voxels 4 * grp .. + 3 of both rows). A workgroup walks bricks with a grid stride; each wave takes two
+// of a brick's eight row pairs and keeps the sums of all 27 taps in registers.
+//
+// Both operands need four consecutive voxels of one channel per lane, so the brick is staged channel by
+// channel: a row of a channel is then read once (12 bytes a lane) for its three x taps, whose
+// fragments are dword-aligned or one 16-bit shift away, instead of eight 2-byte reads per tap and row.
+// The channel strides are 32 bytes past a multiple of 512, so the 64 lanes' 8-byte reads cover every
+// bank once. CIN 4 packs the four channels of four (dz, dy) taps into the 16 rows of A.
+// The waves' sums are added in LDS, and the workgroup writes 27 * CIN * 16 weights, then 16 biases, to
+// partial[block]. 98 x 96 x 91 voxels: 117 -> 33 us a 16-channel layer.
+constexpr int kWgRow = 20;                                   // a row of the input brick: 18 voxels, padded
+constexpr int kWgIn = 36 * kWgRow + 64;                      // a channel: 36 rows; 1568 bytes
+constexpr int kWgOut = BV + 16;                              // a channel of g: 16 rows of 16; 544 bytes
+static_assert((kWgIn * 2) % 512 == 32 && (kWgOut * 2) % 512 == 32, "conflict-free channel strides");
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+// The fragment of two rows (three dwords of six voxels each) at x offset DX - 1.
+template <int DX>
+__device__ inline bf16x8_t wgrad_fragment(const uint32_t (&r0)[3], const uint32_t (&r1)[3])
+{
+	uint4 q;
+	if constexpr (DX == 1) {
+		q = make_uint4(__builtin_amdgcn_alignbit(r0[1], r0[0], 16), __builtin_amdgcn_alignbit(r0[2], r0[1], 16),
+		               __builtin_amdgcn_alignbit(r1[1], r1[0], 16), __builtin_amdgcn_alignbit(r1[2], r1[1], 16));
+	} else {
+		q = make_uint4(r0[DX / 2], r0[DX / 2 + 1], r1[DX / 2], r1[DX / 2 + 1]);
+	}
+	return __builtin_bit_cast(bf16x8_t, q);
+}
+
 template <int CIN>
-__global__ __launch_bounds__(256) void k_conv_wgrad(int nx, int ny, int nz, int nbx, int nby, int nbz,
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad(int nx, int ny, int nz, int nbx, int nby, int nbz,
                                                    const uint16_t *__restrict__ in, const uint16_t *__restrict__ g,
                                                    float *__restrict__ partial)
 {
-	__shared__ __attribute__((aligned(16))) uint16_t lin[HV * CIN];
-	__shared__ __attribute__((aligned(16))) uint16_t lg[BV * 16];
-	__shared__ float dbs[256];
+	constexpr int kParts = CIN / 4;
+	constexpr int kAccs = CIN == 16 ? kCnnTaps : 9;  // CIN 4: (group of four (dz, dy) taps, dx)
+	constexpr int kVals = kCnnTaps * CIN * 16 + 16;
+	constexpr int kStage = (CIN * kWgIn + 16 * kWgOut) * 2, kSums = kVals * 4;
+	__shared__ __attribute__((aligned(16))) uint8_t lds[kStage > kSums ? kStage : kSums];
+	uint16_t *lin = reinterpret_cast<uint16_t *>(lds), *lg = lin + CIN * kWgIn;
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int col = lane & 15, grp = lane >> 4;
-	constexpr int kMyTaps = 7;  // ceil(27 / 4)
-	float4_t acc[kMyTaps];
+	float4_t acc[kAccs], accb = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-	for (int k = 0; k < kMyTaps; ++k) {
+	for (int k = 0; k < kAccs; ++k) {
 		acc[k] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 	}
-	float db = 0.0f;
+	const uint4 one4 = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+	const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, one4);
 	const int nbricks = nbx * nby * nbz;
-	for (int brick = blockIdx.x; brick < nbricks; brick += gridDim.x) {
+	// staging: pairs of x neighbours, four channels each (two 8-byte loads, four dword stores); the loads
+	// of the next brick are in flight while this one is computed
+	constexpr int kInTasks = (HV / 2) * kParts, kOutTasks = (BV / 2) * 4;
+	constexpr int kInIters = (kInTasks + 255) / 256, kOutIters = kOutTasks / 256;
+	uint2 in_lo[kInIters], in_hi[kInIters], out_lo[kOutIters], out_hi[kOutIters];
+	auto fetch = [&](int brick) {
 		const int bx = (brick % nbx) * BX, by = ((brick / nbx) % nby) * BY, bz = (brick / (nbx * nby)) * BZ;
-		__syncthreads();  // the previous brick's LDS reads are done
-		stage_brick<CIN>(lin, in, nx, ny, nz, bx, by, bz);
-		for (int e = threadIdx.x; e < BV * 4; e += blockDim.x) {
-			const int bv = e >> 2, part = e & 3;
-			const int lx = bv % BX, ly = (bv / BX) % BY, lz = bv / (BX * BY);
-			const int x = bx + lx, y = by + ly, z = bz + lz;
-			uint2 val = make_uint2(0u, 0u);
-			if (x < nx && y < ny && z < nz) {
-				const int64_t v = ((int64_t)z * ny + y) * nx + x;
-				val = *reinterpret_cast<const uint2 *>(g + v * 16 + part * 4);
+#pragma unroll
+		for (int i = 0; i < kInIters; ++i) {
+			const int e = (int)threadIdx.x + i * 256;
+			const int part = e % kParts, pv = e / kParts;
+			const int px = pv % (HX / 2), row = pv / (HX / 2);
+			const int x = bx + 2 * px - 1, y = by + row % HY - 1, z = bz + row / HY - 1;
+			const bool in_yz = e < kInTasks && y >= 0 && y < ny && z >= 0 && z < nz;
+			const int64_t v = ((int64_t)z * ny + y) * nx + x;
+			in_lo[i] = in_hi[i] = make_uint2(0u, 0u);
+			if (in_yz && x >= 0 && x < nx) {
+				in_lo[i] = *reinterpret_cast<const uint2 *>(in + v * CIN + part * 4);
 			}
-			*reinterpret_cast<uint2 *>(lg + bv * 16 + part * 4) = val;
+			if (in_yz && x + 1 < nx) {
+				in_hi[i] = *reinterpret_cast<const uint2 *>(in + (v + 1) * CIN + part * 4);
+			}
+		}
+#pragma unroll
+		for (int i = 0; i < kOutIters; ++i) {
+			const int e = (int)threadIdx.x + i * 256;
+			const int part = e & 3, pv = e >> 2;
+			const int px = pv % (BX / 2), row = pv / (BX / 2);
+			const int x = bx + 2 * px, y = by + row % BY, z = bz + row / BY;
+			const int64_t v = ((int64_t)z * ny + y) * nx + x;
+			out_lo[i] = out_hi[i] = make_uint2(0u, 0u);
+			if (y < ny && z < nz && x < nx) {
+				out_lo[i] = *reinterpret_cast<const uint2 *>(g + v * 16 + part * 4);
+			}
+			if (y < ny && z < nz && x + 1 < nx) {
+				out_hi[i] = *reinterpret_cast<const uint2 *>(g + (v + 1) * 16 + part * 4);
+			}
+		}
+	};
+	auto put = [&](uint16_t *to, int stride, uint2 lo, uint2 hi) {
+		*reinterpret_cast<uint32_t *>(to) = (lo.x & 0xffffu) | (hi.x << 16);
+		*reinterpret_cast<uint32_t *>(to + stride) = (lo.x >> 16) | (hi.x & 0xffff0000u);
+		*reinterpret_cast<uint32_t *>(to + 2 * stride) = (lo.y & 0xffffu) | (hi.y << 16);
+		*reinterpret_cast<uint32_t *>(to + 3 * stride) = (lo.y >> 16) | (hi.y & 0xffff0000u);
+	};
+	if ((int)blockIdx.x < nbricks) {
+		fetch(blockIdx.x);
+	}
+	for (int brick = blockIdx.x; brick < nbricks; brick += gridDim.x) {
+		__syncthreads();  // the previous brick's LDS reads are done
+#pragma unroll
+		for (int i = 0; i < kInIters; ++i) {
+			const int e = (int)threadIdx.x + i * 256;
+			const int part = e % kParts, pv = e / kParts;
+			if (e < kInTasks) {
+				put(lin + part * 4 * kWgIn + pv / (HX / 2) * kWgRow + 2 * (pv % (HX / 2)), kWgIn, in_lo[i], in_hi[i]);
+			}
+		}
+#pragma unroll
+		for (int i = 0; i < kOutIters; ++i) {
+			const int e = (int)threadIdx.x + i * 256;
+			const int part = e & 3, pv = e >> 2;
+			put(lg + part * 4 * kWgOut + pv / (BX / 2) * BX + 2 * (pv % (BX / 2)), kWgOut, out_lo[i], out_hi[i]);
 		}
 		__syncthreads();
-		// bias: thread (v16, co) sums 16 voxels of channel co
-		{
-			const int co = threadIdx.x & 15, v16 = threadIdx.x >> 4;
-#pragma unroll
-			for (int k = 0; k < 16; ++k) {
-				db += bf2f(lg[(v16 * 16 + k) * 16 + co]);
-			}
+		if (brick + (int)gridDim.x < nbricks) {
+			fetch(brick + gridDim.x);
 		}
-#pragma unroll
-		for (int k = 0; k < kMyTaps; ++k) {
-			const int t = wave + 4 * k;
-			if (t >= kCnnTaps) {
-				continue;
-			}
 #pragma unroll 1
-			for (int row = 0; row < BY * BZ; ++row) {
-				const int ly = row % BY, lz = row / BY;
-				short4_t av, bv;
+		for (int pair = wave; pair < BY * BZ / 2; pair += 4) {
+			const int ly = (2 * pair) % BY, lz = (2 * pair) / BY;
+			const uint16_t *gr = lg + col * kWgOut + 2 * pair * BX + 4 * grp;
+			const uint2 g0 = *reinterpret_cast<const uint2 *>(gr), g1 = *reinterpret_cast<const uint2 *>(gr + BX);
+			const uint4 gq = make_uint4(g0.x, g0.y, g1.x, g1.y);
+			const bf16x8_t bv = __builtin_bit_cast(bf16x8_t, gq);
+			accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, bv, accb, 0, 0, 0);
+			if constexpr (CIN == 16) {
 #pragma unroll
-				for (int j = 0; j < 4; ++j) {
-					const int x = 4 * grp + j;  // voxel of the chunk (k index)
-					const int hv = ((lz + 1 + tap_dz(t)) * HY + (ly + 1 + tap_dy(t))) * HX + (x + 1 + tap_dx(t));
-					av[j] = col < CIN ? (short)lin[hv * CIN + (col < CIN ? col : 0)] : (short)0;
-					bv[j] = (short)lg[(row * BX + x) * 16 + col];
+				for (int dz = 0; dz < 3; ++dz) {
+					uint32_t r[4][3];  // input rows ly - 1 .. ly + 2 of slice lz + dz - 1, six voxels from 4 * grp - 1
+#pragma unroll
+					for (int i = 0; i < 4; ++i) {
+						const uint16_t *ir = lin + col * kWgIn + ((lz + dz) * HY + ly + i) * kWgRow + 4 * grp;
+						const uint2 q = *reinterpret_cast<const uint2 *>(ir);
+						r[i][0] = q.x;
+						r[i][1] = q.y;
+						r[i][2] = *reinterpret_cast<const uint32_t *>(ir + 4);
+					}
+#pragma unroll
+					for (int dy = 0; dy < 3; ++dy) {
+						const int t = dz * 9 + dy * 3;
+						acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wgrad_fragment<0>(r[dy], r[dy + 1]), bv, acc[t], 0,
+						                                                 0, 0);
+						acc[t + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wgrad_fragment<1>(r[dy], r[dy + 1]), bv,
+						                                                     acc[t + 1], 0, 0, 0);
+						acc[t + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wgrad_fragment<2>(r[dy], r[dy + 1]), bv,
+						                                                     acc[t + 2], 0, 0, 0);
+					}
 				}
-				acc[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[k], 0, 0, 0);
+			} else {
+#pragma unroll
+				for (int m = 0; m < 3; ++m) {
+					const int zy = 4 * m + (col >> 2) < 9 ? 4 * m + (col >> 2) : 8;  // (rows past tap 8 are dropped)
+					uint32_t r[2][3];
+#pragma unroll
+					for (int i = 0; i < 2; ++i) {
+						const uint16_t *ir =
+						    lin + (col & 3) * kWgIn + ((lz + zy / 3) * HY + ly + zy % 3 + i) * kWgRow + 4 * grp;
+						const uint2 q = *reinterpret_cast<const uint2 *>(ir);
+						r[i][0] = q.x;
+						r[i][1] = q.y;
+						r[i][2] = *reinterpret_cast<const uint32_t *>(ir + 4);
+					}
+					acc[3 * m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wgrad_fragment<0>(r[0], r[1]), bv, acc[3 * m], 0,
+					                                                     0, 0);
+					acc[3 * m + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wgrad_fragment<1>(r[0], r[1]), bv,
+					                                                         acc[3 * m + 1], 0, 0, 0);
+					acc[3 * m + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wgrad_fragment<2>(r[0], r[1]), bv,
+					                                                         acc[3 * m + 2], 0, 0, 0);
+				}
 			}
 		}
 	}
-	float *mine = partial + (int64_t)blockIdx.x * (kCnnTaps * CIN * 16 + 16);
-#pragma unroll
-	for (int k = 0; k < kMyTaps; ++k) {
-		const int t = wave + 4 * k;
-		if (t >= kCnnTaps) {
+	// the waves' sums, one after another: D row 4 * grp + j, column col = co
+	float *sums = reinterpret_cast<float *>(lds);
+#pragma unroll 1
+	for (int w = 0; w < 4; ++w) {
+		__syncthreads();
+		if (wave != w) {
 			continue;
 		}
-		// D[ci][co]: lane holds co = col, ci = 4 * grp + j
+		auto add = [&](int i, float v) { sums[i] = w == 0 ? v : sums[i] + v; };
 #pragma unroll
-		for (int j = 0; j < 4; ++j) {
-			const int ci = 4 * grp + j;
-			if (ci < CIN) {
-				mine[(t * CIN + ci) * 16 + col] = acc[k][j];
+		for (int k = 0; k < kAccs; ++k) {
+#pragma unroll
+			for (int j = 0; j < 4; ++j) {
+				if constexpr (CIN == 16) {
+					add((k * 16 + 4 * grp + j) * 16 + col, acc[k][j]);
+				} else {
+					const int zy = 4 * (k / 3) + grp;  // row = 4 * (tap of the group) + channel
+					if (zy < 9) {
+						add(((zy * 3 + k % 3) * 4 + j) * 16 + col, acc[k][j]);
+					}
+				}
 			}
 		}
-	}
-	dbs[threadIdx.x] = db;
-	__syncthreads();
-	if (threadIdx.x < 16) {
-		float s = 0.0f;
-		for (int k = threadIdx.x; k < 256; k += 16) {
-			s += dbs[k];
+		if (grp == 0) {
+			add(kCnnTaps * CIN * 16 + col, accb[0]);
 		}
-		mine[kCnnTaps * CIN * 16 + threadIdx.x] = s;
+	}
+	__syncthreads();
+	float *mine = partial + (int64_t)blockIdx.x * kVals;
+	for (int i = threadIdx.x; i < kVals; i += 256) {
+		mine[i] = sums[i];
 	}
 }
 
-// out[i] = sum over blocks of partial[block][i]
-__global__ __launch_bounds__(256) void k_reduce_partials(const float *__restrict__ partial, int nblocks, int nvals,
-                                                        float *__restrict__ out)
+// out[i] = sum over blocks of partial[block][i]: 64 consecutive values a workgroup, 16 threads a
+// value over the blocks (one thread a value left the chip idle: 27 workgroups in a chain of 2048 loads,
+// 441 us a layer; now 8 us).
+constexpr int kReduceCols = 64, kReduceRows = 16;
+
+__global__ __launch_bounds__(kReduceCols *kReduceRows) void k_reduce_partials(const float *__restrict__ partial,
+                                                                              int nblocks, int nvals,
+                                                                              float *__restrict__ out)
 {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= nvals) {
-		return;
-	}
+	__shared__ float red[kReduceRows][kReduceCols];
+	const int c = threadIdx.x % kReduceCols, r = threadIdx.x / kReduceCols;
+	const int i = blockIdx.x * kReduceCols + c;
 	float s = 0.0f;
-	for (int b = 0; b < nblocks; ++b) {
-		s += partial[(int64_t)b * nvals + i];
+	if (i < nvals) {
+#pragma unroll 8
+		for (int b = r; b < nblocks; b += kReduceRows) {
+			s += partial[(int64_t)b * nvals + i];
+		}
 	}
-	out[i] = s;
+	red[r][c] = s;
+	__syncthreads();
+	if (r == 0 && i < nvals) {
+#pragma unroll
+		for (int k = 1; k < kReduceRows; ++k) {
+			s += red[k][c];
+		}
+		out[i] = s;
+	}
 }
 
 // Head backward: dz = (sigmoid(z) - y) / n; the gradient at layer 4's pre-activation is
-// dz * w_head where layer 4's output is positive. Per-block partials: dw_head[16], then
-// (double accumulators) loss and db_head.
+// dz * w_head where layer 4's output is positive. Per-block partials: dw_head[16], and loss and
+// db_head in double.
 __global__ __launch_bounds__(256) void k_head_bwd(int64_t n, const float *__restrict__ logits,
                                                  const uint8_t *__restrict__ label, const uint16_t *__restrict__ act,
                                                  const float *__restrict__ head, uint16_t *__restrict__ g,
-                                                 float *__restrict__ partial, double *__restrict__ scalars)
+                                                 float *__restrict__ partial, double2 *__restrict__ scalars)
 {
-	__shared__ float red[16][257];
-	__shared__ double rl[256], rb[256];
+	__shared__ float red[4][16];
+	__shared__ double rl[4], rb[4];
 	const float inv_n = 1.0f / (float)n;
 	float gw[16];
 #pragma unroll
@@ -551,45 +665,74 @@ __global__ __launch_bounds__(256) void k_head_bwd(int64_t n, const float *__rest
 		const float dz = (p - y) * inv_n;
 		loss += (double)(fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))) - y * z);
 		dbh += (double)dz;
-		uint16_t out[16];
+		const uint4 *from = reinterpret_cast<const uint4 *>(act + v * 16);
+		uint4 q[2] = {from[0], from[1]};
+		uint16_t *a16 = reinterpret_cast<uint16_t *>(q);
 #pragma unroll
 		for (int c = 0; c < 16; ++c) {
-			const float a = bf2f(act[v * 16 + c]);
+			const float a = bf2f(a16[c]);
 			gw[c] += dz * a;
-			out[c] = a > 0.0f ? f2bf(dz * head[c]) : 0;
+			a16[c] = a > 0.0f ? f2bf(dz * head[c]) : 0;
 		}
+		uint4 *to = reinterpret_cast<uint4 *>(g + v * 16);
+		to[0] = q[0];
+		to[1] = q[1];
+	}
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-		for (int c = 0; c < 16; c += 4) {
-			ushort4 q;
-			q.x = out[c];
-			q.y = out[c + 1];
-			q.z = out[c + 2];
-			q.w = out[c + 3];
-			*reinterpret_cast<ushort4 *>(g + v * 16 + c) = q;
+	for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+		for (int c = 0; c < 16; ++c) {
+			gw[c] += __shfl_xor(gw[c], off, 64);
 		}
+		loss += __shfl_xor(loss, off, 64);
+		dbh += __shfl_xor(dbh, off, 64);
 	}
+	if (lane == 0) {
 #pragma unroll
-	for (int c = 0; c < 16; ++c) {
-		red[c][threadIdx.x] = gw[c];
+		for (int c = 0; c < 16; ++c) {
+			red[wave][c] = gw[c];
+		}
+		rl[wave] = loss;
+		rb[wave] = dbh;
 	}
-	rl[threadIdx.x] = loss;
-	rb[threadIdx.x] = dbh;
 	__syncthreads();
 	if (threadIdx.x < 16) {
-		float s = 0.0f;
-		for (int k = 0; k < 256; ++k) {
-			s += red[threadIdx.x][k];
-		}
-		partial[(int64_t)blockIdx.x * 16 + threadIdx.x] = s;
+		const int c = threadIdx.x;
+		partial[(int64_t)blockIdx.x * 16 + c] = red[0][c] + red[1][c] + red[2][c] + red[3][c];
 	}
 	if (threadIdx.x == 0) {
-		double a = 0.0, b = 0.0;
-		for (int k = 0; k < 256; ++k) {
-			a += rl[k];
-			b += rb[k];
-		}
-		atomicAdd(&scalars[0], a);
-		atomicAdd(&scalars[1], b);
+		scalars[1 + blockIdx.x] = make_double2(rl[0] + rl[1] + rl[2] + rl[3], rb[0] + rb[1] + rb[2] + rb[3]);
+	}
+}
+
+// scalars[0] = sum of the blocks' (loss, db_head); db_head also goes to its place in the gradient. (An
+// atomic per block on the two words held the head's kernel up: 71 -> 16 us with its wave sums.)
+__global__ __launch_bounds__(256) void k_sum_scalars(double2 *__restrict__ scalars, int nblocks,
+                                                    float *__restrict__ head_bias)
+{
+	__shared__ double rl[4], rb[4];
+	double a = 0.0, b = 0.0;
+	for (int i = threadIdx.x; i < nblocks; i += 256) {
+		const double2 q = scalars[1 + i];
+		a += q.x;
+		b += q.y;
+	}
+#pragma unroll
+	for (int off = 32; off > 0; off >>= 1) {
+		a += __shfl_xor(a, off, 64);
+		b += __shfl_xor(b, off, 64);
+	}
+	if ((threadIdx.x & 63) == 0) {
+		rl[threadIdx.x >> 6] = a;
+		rb[threadIdx.x >> 6] = b;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		a = rl[0] + rl[1] + rl[2] + rl[3];
+		b = rb[0] + rb[1] + rb[2] + rb[3];
+		scalars[0] = make_double2(a, b);
+		*head_bias = (float)b;
 	}
 }
 
@@ -647,7 +790,6 @@ CnnModel::CnnModel(hipStream_t stream) : mStream(stream), mHost(kCnnParams, 0.0f
 	mAdamV.allocate(kCnnParams);
 	mPackFwd.allocate(kPackFwd);
 	mPackBwd.allocate(kPackBwd);
-	mScalars.allocate(2);
 	CGP_HIP(hipMemsetAsync(mParams.get(), 0, kCnnParams * sizeof(float), mStream));
 	CGP_HIP(hipMemsetAsync(mAdamM.get(), 0, kCnnParams * sizeof(float), mStream));
 	CGP_HIP(hipMemsetAsync(mAdamV.get(), 0, kCnnParams * sizeof(float), mStream));
@@ -771,25 +913,30 @@ void CnnModel::run_backward(GridSolver &grid, double &loss)
 {
 	const uint8_t *label = grid.device_source_side(0);
 	const float *p = mParams.get();
-	CGP_HIP(hipMemsetAsync(mScalars.get(), 0, 2 * sizeof(double), mStream));
-	const int head_blocks = blocks_of(mVox, 2048);
+	// a few workgroups per CU, each over several bricks: fewer partial sums to write and add up
+	const int head_blocks = blocks_of(mVox, 1024);
 	const int nbx = (mNx + BX - 1) / BX, nby = (mNy + BY - 1) / BY, nbz = (mNz + BZ - 1) / BZ;
-	const int wg_blocks = std::min(nbx * nby * nbz, 2048);
+	const int wg_blocks = std::min(nbx * nby * nbz, 512);
 	const int per16 = kCnnTaps * 16 * 16 + 16, per4 = kCnnTaps * 4 * 16 + 16;
 	mPartials.allocate((size_t)std::max(head_blocks * 16, wg_blocks * per16));
+	mScalars.allocate((size_t)head_blocks + 1);
+	const auto reduce = [&](int nblocks, int nvals, float *out) {
+		hipLaunchKernelGGL(k_reduce_partials, dim3((nvals + kReduceCols - 1) / kReduceCols),
+		                   dim3(kReduceCols * kReduceRows), 0, mStream, mPartials.get(), nblocks, nvals, out);
+	};
 	// head
 	hipLaunchKernelGGL(k_head_bwd, dim3(head_blocks), dim3(256), 0, mStream, mVox, mLogit.get(), label, mAct[3].get(),
 	                   p + kOffHeadW, mG[0].get(), mPartials.get(), mScalars.get());
-	hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, mStream, mPartials.get(), head_blocks, 16,
-	                   mGrad.get() + kOffHeadW);
+	hipLaunchKernelGGL(k_sum_scalars, dim3(1), dim3(256), 0, mStream, mScalars.get(), head_blocks,
+	                   mGrad.get() + kOffHeadB);
+	reduce(head_blocks, 16, mGrad.get() + kOffHeadW);
 	const dim3 grid3(nbx, nby, nbz);
 	int cur = 0;
 	for (int layer = 3; layer >= 1; --layer) {
 		// weight gradient of `layer` (input: activation of layer - 1, gradient at its pre-activation in mG[cur])
 		hipLaunchKernelGGL((k_conv_wgrad<16>), dim3(wg_blocks), dim3(256), 0, mStream, mNx, mNy, mNz, nbx, nby, nbz,
 		                   mAct[layer - 1].get(), mG[cur].get(), mPartials.get());
-		hipLaunchKernelGGL(k_reduce_partials, dim3((per16 + 255) / 256), dim3(256), 0, mStream, mPartials.get(),
-		                   wg_blocks, per16, mGrad.get() + off_w(layer));
+		reduce(wg_blocks, per16, mGrad.get() + off_w(layer));
 		// gradient at the pre-activation of layer - 1
 		hipLaunchKernelGGL((k_conv<16, true, false>), grid3, dim3(256), 0, mStream, mNx, mNy, mNz, mG[cur].get(),
 		                   mPackBwd.get() + (layer - 1) * kPackL, (const float *)nullptr, mAct[layer - 1].get(),
@@ -798,16 +945,12 @@ void CnnModel::run_backward(GridSolver &grid, double &loss)
 	}
 	hipLaunchKernelGGL((k_conv_wgrad<4>), dim3(wg_blocks), dim3(256), 0, mStream, mNx, mNy, mNz, nbx, nby, nbz,
 	                   mX0.get(), mG[cur].get(), mPartials.get());
-	hipLaunchKernelGGL(k_reduce_partials, dim3((per4 + 255) / 256), dim3(256), 0, mStream, mPartials.get(), wg_blocks,
-	                   per4, mGrad.get() + kOffW1);
+	reduce(wg_blocks, per4, mGrad.get() + kOffW1);
 	CGP_LAUNCH_CHECK();
-	double host[2];
-	CGP_HIP(hipMemcpyAsync(host, mScalars.get(), sizeof(host), hipMemcpyDeviceToHost, mStream));
+	double host = 0.0;
+	CGP_HIP(hipMemcpyAsync(&host, mScalars.get(), sizeof(host), hipMemcpyDeviceToHost, mStream));
 	CGP_HIP(hipStreamSynchronize(mStream));
-	const float dbh = (float)host[1];
-	CGP_HIP(hipMemcpyAsync(mGrad.get() + kOffHeadB, &dbh, sizeof(float), hipMemcpyHostToDevice, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
-	loss = host[0] / (double)mVox;
+	loss = host / (double)mVox;
 }
 
 double CnnModel::gradients(GridSolver &grid, const uint8_t *volume, bool device_volume, float *grad)

@@ -30,9 +30,9 @@ public:
 	explicit CnnModel(hipStream_t stream);
 	void set_params(const float *params);
 	void get_params(float *params);
-	// Forward on grid 0 of `grid` with the given volume (host or device bytes). Keeps the logits and,
-	// if `keep_activations`, every layer's activations for a backward pass.
-	void forward(GridSolver &grid, const uint8_t *volume, bool device_volume, bool keep_activations);
+	// Forward on grid 0 of `grid` with the given volume (host or device bytes). Keeps the logits, the
+	// thresholded side and every layer's activations; `wait`: until they are there.
+	void forward(GridSolver &grid, const uint8_t *volume, bool device_volume, bool wait);
 	// Thresholded prediction (logit > 0) as a 0/1 byte mask in device memory of the grid's size.
 	const uint8_t *predicted_side();
 	void prediction_to_host(uint8_t *side, float *prob);
@@ -61,7 +61,6 @@ private:
 	DeviceBuffer<uint8_t> mVolume, mSide;
 	DeviceBuffer<double2> mScalars;               // loss and head-bias gradient: the sum, then per-block sums
 	int mStep = 0;
-	bool mPackDirty = true;
 };
 
 }  // namespace cgp

@@ -235,11 +235,9 @@ __global__ __launch_bounds__(256) void k_conv(int nx, int ny, int nz, const uint
 	}
 }
 
-// Forward layer for inference, marching along z: workgroup (bx, by, bz) computes kZBricks
-// consecutive 16 x 4 x 4 output bricks in z. The input planes stay in an LDS ring of 8 z-planes
+// Forward layer, marching along z: workgroup (bx, by, bz) computes zbricks (z_bricks below) consecutive 16 x 4 x 4 output bricks in z. The input planes stay in an LDS ring of 8 z-planes
 // (one plane per 4-channel group as in k_conv), so each brick stages only the 4 planes it adds
 // instead of its whole 6-plane halo box. Same arithmetic and output as k_conv<CIN, false, HEAD>.
-constexpr int kZBricks = 8;
 constexpr int kZSlots = 8;
 
 // Per-thread staging map of one input z-plane of the brick box (18 x 6 voxels, CIN / 4 channel
@@ -295,12 +293,12 @@ template <int CIN, bool HEAD>
 __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, const uint16_t *__restrict__ in,
                                                    const uint16_t *__restrict__ pack, const float *__restrict__ bias,
                                                    uint16_t *__restrict__ out, const float *__restrict__ head,
-                                                   float *__restrict__ logits)
+                                                   float *__restrict__ logits, int zbricks)
 {
 	static_assert(kZSlots == 8, "ring slots are taken modulo 8");
 	constexpr int PL = HX * HY;
 	__shared__ __attribute__((aligned(16))) uint16_t lds[kZSlots * PL * CIN];
-	const int bx = blockIdx.x * BX, by = blockIdx.y * BY, bz0 = blockIdx.z * (kZBricks * BZ);
+	const int bx = blockIdx.x * BX, by = blockIdx.y * BY, bz0 = blockIdx.z * (zbricks * BZ);
 	constexpr int NM = CIN == 16 ? 27 : 7;
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int col = lane & 15, grp = lane >> 4;
@@ -326,7 +324,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, cons
 	// the lane's LDS base: its channel group's planes, its voxel column (x + 1 for the halo)
 	const uint32_t lbase = (uint32_t)((((CIN == 16 ? grp : 0) * kZSlots * PL) + col + 1) * 4);
 	const int lz = wave;
-	for (int zb = 0; zb < kZBricks; ++zb) {
+	for (int zb = 0; zb < zbricks; ++zb) {
 		const int bz = bz0 + zb * BZ;
 		if (bz >= nz) {
 			break;  // uniform across the workgroup
@@ -774,6 +772,18 @@ __global__ __launch_bounds__(256) void k_sigmoid(int64_t n, const float *__restr
 	}
 }
 
+// Bricks a workgroup of the forward layers marches: long marches stage fewer halo planes, short ones
+// fill the chip. Five workgroups fit a CU (LDS), so 8 bricks need some 2500 workgroups to keep the last
+// ones from running alone, and below 512 half the CUs idle. 16 -> 16 layer with 8 / 6 / 4 / 2 / 1 bricks:
+// 131 x 125 x 119 voxels 59 / 71 / 59 / 66 / 72 us (with the head 81 / 78 / 70 / 76 / 85),
+// 98 x 96 x 91: 44 / 37 / 31 / 32 / 35 us.
+int z_bricks(int nx, int ny, int nz)
+{
+	const int64_t columns = (int64_t)((nx + BX - 1) / BX) * ((ny + BY - 1) / BY);
+	const auto groups = [&](int bricks) { return columns * ((nz + BZ * bricks - 1) / (BZ * bricks)); };
+	return groups(8) >= 2560 ? 8 : groups(4) >= 512 ? 4 : groups(2) >= 512 ? 2 : 1;
+}
+
 int blocks_of(int64_t n, int cap = 8192)
 {
 	int64_t b = (n + 255) / 256;
@@ -848,7 +858,7 @@ void CnnModel::ensure(int64_t vox)
 	mVox = vox;
 }
 
-void CnnModel::forward(GridSolver &grid, const uint8_t *volume, bool device_volume, bool)
+void CnnModel::forward(GridSolver &grid, const uint8_t *volume, bool device_volume, bool wait)
 {
 	if (!volume) {
 		volume = grid.device_volume();  // the grid was built from its volume on the device
@@ -868,22 +878,25 @@ void CnnModel::forward(GridSolver &grid, const uint8_t *volume, bool device_volu
 		vol = mVolume.get();
 	}
 	hipLaunchKernelGGL(k_cnn_input, dim3(blocks_of(mVox)), dim3(256), 0, mStream, mVox, vol, d.cs, d.ct, mX0.get());
-	// inference layers march along z, kZBricks bricks a workgroup
-	const dim3 gridz((mNx + BX - 1) / BX, (mNy + BY - 1) / BY, (mNz + BZ * kZBricks - 1) / (BZ * kZBricks));
+	// the layers march along z, zbricks bricks a workgroup
+	const int zbricks = z_bricks(mNx, mNy, mNz);
+	const dim3 gridz((mNx + BX - 1) / BX, (mNy + BY - 1) / BY, (mNz + BZ * zbricks - 1) / (BZ * zbricks));
 	const float *p = mParams.get();
 	hipLaunchKernelGGL((k_conv_fwd_z<4, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mX0.get(),
 	                   mPackFwd.get() + pack_fwd_off(0), p + off_b(0), mAct[0].get(), (const float *)nullptr,
-	                   (float *)nullptr);
+	                   (float *)nullptr, zbricks);
 	for (int layer = 1; layer <= 2; ++layer) {
 		hipLaunchKernelGGL((k_conv_fwd_z<16, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz,
 		                   mAct[layer - 1].get(), mPackFwd.get() + pack_fwd_off(layer), p + off_b(layer),
-		                   mAct[layer].get(), (const float *)nullptr, (float *)nullptr);
+		                   mAct[layer].get(), (const float *)nullptr, (float *)nullptr, zbricks);
 	}
 	hipLaunchKernelGGL((k_conv_fwd_z<16, true>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mAct[2].get(),
-	                   mPackFwd.get() + pack_fwd_off(3), p + off_b(3), mAct[3].get(), p + kOffHeadW, mLogit.get());
+	                   mPackFwd.get() + pack_fwd_off(3), p + off_b(3), mAct[3].get(), p + kOffHeadW, mLogit.get(), zbricks);
 	hipLaunchKernelGGL(k_threshold, dim3(blocks_of(mVox)), dim3(256), 0, mStream, mVox, mLogit.get(), mSide.get());
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipStreamSynchronize(mStream));
+	if (wait) {
+		CGP_HIP(hipStreamSynchronize(mStream));
+	}
 }
 
 const uint8_t *CnnModel::predicted_side()
@@ -955,7 +968,7 @@ void CnnModel::run_backward(GridSolver &grid, double &loss)
 
 double CnnModel::gradients(GridSolver &grid, const uint8_t *volume, bool device_volume, float *grad)
 {
-	forward(grid, volume, device_volume, true);
+	forward(grid, volume, device_volume, false);  // the backward pass follows on the same stream
 	double loss = 0.0;
 	run_backward(grid, loss);
 	if (grad) {

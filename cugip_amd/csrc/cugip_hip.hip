@@ -557,7 +557,7 @@ int cgp_cnn_predict(cgp_cnn c, cgp_graph g, const uint8_t *volume, uint8_t *side
 {
 	return cnn_guarded(c, [&] {
 		cgp::GridSolver &grid = cnn_grid(g);
-		c->model->forward(grid, volume, false, false);
+		c->model->forward(grid, volume, false, true);
 		c->model->prediction_to_host(side, prob);
 		if (certificate) {
 			*certificate = grid.cut_capacity_device(0, c->model->predicted_side());

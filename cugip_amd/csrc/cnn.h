@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "common.h"
+#include "host_copy.h"
 
 namespace cgp {
 
@@ -49,6 +50,7 @@ private:
 	void run_backward(GridSolver &grid, double &loss);
 
 	hipStream_t mStream;
+	HostCopier mCopier;
 	int mNx = 0, mNy = 0, mNz = 0;
 	int64_t mVox = 0;
 	std::vector<float> mHost;                     // fp32 master parameters (host mirror)
@@ -57,7 +59,7 @@ private:
 	DeviceBuffer<uint16_t> mX0;                   // input, 4 channels
 	DeviceBuffer<uint16_t> mAct[4];               // post-ReLU activations of the 4 conv layers
 	DeviceBuffer<uint16_t> mG[2];                 // pre-activation gradients (ping-pong)
-	DeviceBuffer<float> mLogit;
+	DeviceBuffer<float> mLogit, mProb;
 	DeviceBuffer<uint8_t> mVolume, mSide;
 	DeviceBuffer<double2> mScalars;               // loss and head-bias gradient: the sum, then per-block sums
 	int mStep = 0;

@@ -910,16 +910,14 @@ const uint8_t *CnnModel::predicted_side()
 void CnnModel::prediction_to_host(uint8_t *side, float *prob)
 {
 	if (side) {
-		CGP_HIP(hipMemcpyAsync(side, mSide.get(), mVox, hipMemcpyDeviceToHost, mStream));
+		mCopier.read(side, mSide.get(), mVox, mStream);
 	}
 	if (prob) {
-		DeviceBuffer<float> p(mVox);
-		hipLaunchKernelGGL(k_sigmoid, dim3(blocks_of(mVox)), dim3(256), 0, mStream, mVox, mLogit.get(), p.get());
+		mProb.allocate(mVox);
+		hipLaunchKernelGGL(k_sigmoid, dim3(blocks_of(mVox)), dim3(256), 0, mStream, mVox, mLogit.get(), mProb.get());
 		CGP_LAUNCH_CHECK();
-		CGP_HIP(hipMemcpyAsync(prob, p.get(), mVox * sizeof(float), hipMemcpyDeviceToHost, mStream));
-		CGP_HIP(hipStreamSynchronize(mStream));
+		mCopier.read(prob, mProb.get(), mVox * sizeof(float), mStream);
 	}
-	CGP_HIP(hipStreamSynchronize(mStream));
 }
 
 void CnnModel::run_backward(GridSolver &grid, double &loss)
@@ -972,8 +970,7 @@ double CnnModel::gradients(GridSolver &grid, const uint8_t *volume, bool device_
 	double loss = 0.0;
 	run_backward(grid, loss);
 	if (grad) {
-		CGP_HIP(hipMemcpyAsync(grad, mGrad.get(), kCnnParams * sizeof(float), hipMemcpyDeviceToHost, mStream));
-		CGP_HIP(hipStreamSynchronize(mStream));
+		mCopier.read(grad, mGrad.get(), kCnnParams * sizeof(float), mStream);
 		for (int t = 0; t < kCnnTaps; ++t) {
 			for (int co = 0; co < kCnnChannels; ++co) {
 				grad[kOffW1 + (t * 4 + 3) * kCnnChannels + co] = 0.0f;  // padding channel

@@ -139,7 +139,7 @@ void CsrSolver::set_nweights(int m, const cgp_edge *edges, const int32_t *fwd, c
 	mSolved = false;
 	mHeadroomChecked = false;
 	mFirst.allocate(mN + 1);
-	CGP_HIP(hipMemcpyAsync(mFirst.get(), mHostFirst.data(), (mN + 1) * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
+	CGP_HIP(hipMemcpyAsync(mFirst.get(), mHostFirst.data(), ((size_t)mN + 1) * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
 	if (arcs > 0) {
 		mEnds.allocate(arcs);
 		mCap.allocate(arcs);
@@ -169,8 +169,8 @@ void CsrSolver::set_tweights(const int32_t *source, const int32_t *sink)
 		}
 	}
 	mHostSource.assign(source, source + mN);
-	CGP_HIP(hipMemcpyAsync(mCs.get(), source, mN * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
-	CGP_HIP(hipMemcpyAsync(mCt.get(), sink, mN * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
+	CGP_HIP(hipMemcpyAsync(mCs.get(), source, (size_t)mN * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
+	CGP_HIP(hipMemcpyAsync(mCt.get(), sink, (size_t)mN * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
 	CGP_HIP(hipStreamSynchronize(mStream));
 	mHaveTweights = true;
 	mHeadroomChecked = false;
@@ -365,8 +365,7 @@ void CsrSolver::sink_side(uint8_t *host_out, uint8_t mask, uint8_t background)
 	hipLaunchKernelGGL(k_csr_masks, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mH.get(), mS.get(), mMask.get(), 0,
 	                   mask, background);
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipMemcpyAsync(host_out, mMask.get(), mN, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(host_out, mMask.get(), mN, mStream);
 }
 
 void CsrSolver::source_side(uint8_t *host_out)
@@ -377,8 +376,7 @@ void CsrSolver::source_side(uint8_t *host_out)
 	hipLaunchKernelGGL(k_csr_masks, dim3(grid_blocks(mN)), dim3(256), 0, mStream, mN, mH.get(), mS.get(), mMask.get(), 1,
 	                   (uint8_t)1, (uint8_t)0);
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipMemcpyAsync(host_out, mMask.get(), mN, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(host_out, mMask.get(), mN, mStream);
 }
 
 void CsrSolver::labels(int32_t *host_out)
@@ -386,8 +384,7 @@ void CsrSolver::labels(int32_t *host_out)
 	if (!mSolved) {
 		fail(CGP_ERR_STATE, "labels before max_flow");
 	}
-	CGP_HIP(hipMemcpyAsync(host_out, mH.get(), mN * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(host_out, mH.get(), (size_t)mN * sizeof(int32_t), mStream);
 }
 
 }  // namespace cgp

@@ -418,12 +418,11 @@ void GridSolver::capacities(int index, int32_t *cs, int32_t *ct, int32_t *cn, in
 	const InstanceDesc &d = instance(index);
 	const int half = mConn / 2;
 	const size_t vb = (size_t)d.nvox * sizeof(int32_t);
-	CGP_HIP(hipMemcpyAsync(cs, mCs.get() + d.vbase, vb, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipMemcpyAsync(ct, mCt.get() + d.vbase, vb, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipMemcpyAsync(cn, mCn.get() + d.vbase * half, vb * half, hipMemcpyDeviceToHost, mStream));
+	mCopier.read(cs, mCs.get() + d.vbase, vb, mStream);
+	mCopier.read(ct, mCt.get() + d.vbase, vb, mStream);
+	mCopier.read(cn, mCn.get() + d.vbase * half, vb * half, mStream);
 	const int32_t *back = mHasBack ? mCnb.get() : mCn.get();
-	CGP_HIP(hipMemcpyAsync(cnb, back + d.vbase * half, vb * half, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(cnb, back + d.vbase * half, vb * half, mStream);
 }
 
 const InstanceDesc &GridSolver::instance(int index) const
@@ -1459,12 +1458,13 @@ void GridSolver::sink_side(int index, uint8_t *host_out, uint8_t mask, uint8_t b
 	}
 	ensure_exact_labels();
 	const InstanceDesc &d = instance(index);
-	DeviceBuffer<uint8_t> tmp(d.nvox);
+	if ((int64_t)mMask.size() < d.nvox) {
+		mMask.allocate(d.nvox);
+	}
 	hipLaunchKernelGGL(k_sink_side_mask, dim3(blocks_for(d.nvox, 256, 8192)), dim3(256), 0, mStream,
-	                   mH.get() + d.vbase, d.nvox, tmp.get(), mask, background);
+	                   mH.get() + d.vbase, d.nvox, mMask.get(), mask, background);
 	CGP_LAUNCH_CHECK();
-	CGP_HIP(hipMemcpyAsync(host_out, tmp.get(), d.nvox, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(host_out, mMask.get(), d.nvox, mStream);
 }
 
 void GridSolver::source_side(int index, uint8_t *host_out)
@@ -1473,8 +1473,7 @@ void GridSolver::source_side(int index, uint8_t *host_out)
 		fail(CGP_ERR_STATE, "source_set before max_flow");
 	}
 	const InstanceDesc &d = instance(index);
-	CGP_HIP(hipMemcpyAsync(host_out, mS.get() + d.vbase, d.nvox, hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(host_out, mS.get() + d.vbase, d.nvox, mStream);
 }
 
 void GridSolver::source_side_device(int index, uint8_t *out)
@@ -1494,8 +1493,7 @@ void GridSolver::labels(int index, int32_t *host_out)
 	}
 	ensure_exact_labels();
 	const InstanceDesc &d = instance(index);
-	CGP_HIP(hipMemcpyAsync(host_out, mH.get() + d.vbase, d.nvox * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
-	CGP_HIP(hipStreamSynchronize(mStream));
+	mCopier.read(host_out, mH.get() + d.vbase, d.nvox * sizeof(int32_t), mStream);
 }
 
 void GridSolver::state(int index, int32_t *excess, int32_t *labels, uint32_t *saturated)
@@ -1505,7 +1503,7 @@ void GridSolver::state(int index, int32_t *excess, int32_t *labels, uint32_t *sa
 	}
 	const InstanceDesc &d = instance(index);
 	if (excess) {
-		CGP_HIP(hipMemcpyAsync(excess, mE.get() + d.vbase, d.nvox * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
+		mCopier.read(excess, mE.get() + d.vbase, d.nvox * sizeof(int32_t), mStream);
 	}
 	if (saturated) {
 		DeviceBuffer<uint32_t> bits(d.nvox);
@@ -1522,16 +1520,14 @@ void GridSolver::state(int index, int32_t *excess, int32_t *labels, uint32_t *sa
 			                   bits.get());
 		}
 		CGP_LAUNCH_CHECK();
-		CGP_HIP(hipMemcpyAsync(saturated, bits.get(), d.nvox * sizeof(uint32_t), hipMemcpyDeviceToHost, mStream));
-		CGP_HIP(hipStreamSynchronize(mStream));
+		mCopier.read(saturated, bits.get(), d.nvox * sizeof(uint32_t), mStream);
 	}
 	if (labels) {
 		if (mSolved) {
 			ensure_exact_labels();
 		}
-		CGP_HIP(hipMemcpyAsync(labels, mH.get() + d.vbase, d.nvox * sizeof(int32_t), hipMemcpyDeviceToHost, mStream));
+		mCopier.read(labels, mH.get() + d.vbase, d.nvox * sizeof(int32_t), mStream);
 	}
-	CGP_HIP(hipStreamSynchronize(mStream));
 }
 
 void GridSolver::residuals(int index, int32_t *r, int32_t *rt)
@@ -1541,14 +1537,11 @@ void GridSolver::residuals(int index, int32_t *r, int32_t *rt)
 	}
 	const InstanceDesc &d = instance(index);
 	if (r) {
-		CGP_HIP(hipMemcpyAsync(r, mR.get() + d.vbase * mConn, (size_t)d.nvox * mConn * sizeof(int32_t),
-		                       hipMemcpyDeviceToHost, mStream));
+		mCopier.read(r, mR.get() + d.vbase * mConn, (size_t)d.nvox * mConn * sizeof(int32_t), mStream);
 	}
 	if (rt) {
-		CGP_HIP(hipMemcpyAsync(rt, mRt.get() + d.vbase, (size_t)d.nvox * sizeof(int32_t), hipMemcpyDeviceToHost,
-		                       mStream));
+		mCopier.read(rt, mRt.get() + d.vbase, (size_t)d.nvox * sizeof(int32_t), mStream);
 	}
-	CGP_HIP(hipStreamSynchronize(mStream));
 }
 
 GridSolver::DeviceGrid GridSolver::device_grid(int index) const

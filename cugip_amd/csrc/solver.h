@@ -9,6 +9,7 @@
 #include "csr_control.h"
 #include "grid_control.h"
 #include "grid_tile.h"
+#include "host_copy.h"
 
 namespace cgp {
 
@@ -173,6 +174,8 @@ private:
 	                    const GridSpec *borrow = nullptr);
 
 	hipStream_t mStream;
+	HostCopier mCopier;
+	DeviceBuffer<uint8_t> mMask;  // masks on their way to the host, kept between read-backs
 	Arena *mArena = nullptr;  // no-alloc mode: every device buffer is a piece of this block
 	int mNx = 0, mNy = 0, mNz = 0, mConn = 0;  // dimensions of a single grid (instance 0)
 	int64_t mVox = 0;                          // voxels of all instances
@@ -302,6 +305,7 @@ private:
 	const CsrControl &run_stages(int32_t stages, int32_t max_rounds);
 
 	hipStream_t mStream;
+	HostCopier mCopier;
 	int mN = 0;
 	int64_t mArcs = 0;
 	bool mSolved = false;

@@ -54,6 +54,78 @@ __device__ inline int discharge_tile(const int32_t *list, const int32_t *count, 
 }
 
 // ---------------------------------------------------------------------------------------------
+// Tile tables of a single grid: the colour of every tile and the tile ids grouped by colour (each
+// group in tile order, the groups' sizes after the last), for the discharge phases (2 face-parity
+// colours, or 8 of the parities per axis) and for the sweeps (face parity). A tile's place in its group
+// is the number of tiles of its colour before it, which has a closed form. Made on the device because
+// a caller that brings a new grid with every call pays for them: built on the host and copied up they
+// took 43 of the 338 us of a 33 x 30 x 28 no-allocation solve, 111 of the 541 us of 118 x 110 x 105.
+
+// Tiles of face parity c among those before (tx, ty, tz) in tile order. A row has ntx / 2 tiles of each
+// parity and, if ntx is odd, one more of the parity it starts with; planes and rows go the same way.
+__host__ __device__ inline int face_parity_before(int ntx, int nty, int tx, int ty, int tz, int c)
+{
+	int rows_starting = tz * (nty >> 1) + ((ty + ((tz & 1) == c ? 1 : 0)) >> 1);
+	if (nty & 1) {
+		rows_starting += (tz + (c == 0 ? 1 : 0)) >> 1;
+	}
+	const int rows = tz * nty + ty;
+	return rows * (ntx >> 1) + ((ntx & 1) ? rows_starting : 0) + ((tx + (((ty + tz) & 1) == c ? 1 : 0)) >> 1);
+}
+
+__host__ inline int face_parity_tiles(int ntx, int nty, int ntz, int c)
+{
+	return face_parity_before(ntx, nty, 0, 0, ntz, c);
+}
+
+// Indices below n of parity p.
+__host__ __device__ inline int parity_count(int n, int p) { return (n + (p == 0 ? 1 : 0)) >> 1; }
+
+__host__ inline int axis_parity_tiles(int ntx, int nty, int ntz, int c)
+{
+	return parity_count(ntx, c & 1) * parity_count(nty, (c >> 1) & 1) * parity_count(ntz, c >> 2);
+}
+
+struct TileTables {
+	int ntx, nty, ntz, phase_colours;
+	uint8_t *phase_colour, *sweep_colour;
+	int32_t *phase_tiles, *sweep_tiles;
+	int32_t phase_start[8], phase_size[8], sweep_start[2], sweep_size[2];
+};
+
+__global__ __launch_bounds__(256) void k_tile_tables(TileTables out, int32_t *__restrict__ cursors, int cursor_words)
+{
+	const int n = out.ntx * out.nty * out.ntz;
+	const int start = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+	if (start < cursor_words) {
+		cursors[start] = 0;
+	}
+	if (start < out.phase_colours) {
+		out.phase_tiles[n + start] = out.phase_size[start];
+	}
+	if (start < 2) {
+		out.sweep_tiles[n + start] = out.sweep_size[start];
+	}
+	for (int64_t i = start; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+		const int t = (int)i;
+		const int tx = t % out.ntx, ty = (t / out.ntx) % out.nty, tz = t / (out.ntx * out.nty);
+		const int f = (tx + ty + tz) & 1;
+		const int before = face_parity_before(out.ntx, out.nty, tx, ty, tz, f);
+		out.sweep_colour[t] = (uint8_t)f;
+		out.sweep_tiles[out.sweep_start[f] + before] = t;
+		if (out.phase_colours == 2) {
+			out.phase_colour[t] = (uint8_t)f;
+			out.phase_tiles[out.phase_start[f] + before] = t;
+		} else {
+			const int c = (tx & 1) | ((ty & 1) << 1) | ((tz & 1) << 2);
+			const int nxc = parity_count(out.ntx, tx & 1), nyc = parity_count(out.nty, ty & 1);
+			out.phase_colour[t] = (uint8_t)c;
+			out.phase_tiles[out.phase_start[c] + ((tz >> 1) * nyc + (ty >> 1)) * nxc + (tx >> 1)] = t;
+		}
+	}
+}
+
+// ---------------------------------------------------------------------------------------------
 // init: residual planes, cancellation, excess, residual sink link. Sets status bit 0 for a negative
 // capacity, bit 1 when a voxel's inflow or an edge's capacity pair does not fit int32, and bit 2
 // when some edge's capacity pair exceeds 32767 (then residuals cannot be staged as int16).

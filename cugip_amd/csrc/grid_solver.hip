@@ -340,8 +340,7 @@ void GridSolver::set_grid_volume(int nx, int ny, int nz, int conn, const uint8_t
 	}
 	allocate_grids(conn, inst, false);
 	const int64_t n = inst[0].nvox;
-	DeviceBuffer<uint8_t> mark;
-	DeviceBuffer<cgp_volume_weights> w(1);
+	mWeights.allocate(1);
 	const uint8_t *dm = markers;
 	// the volume stays on the device (the learned cut proposal reads it)
 	mVolume.allocate(n);
@@ -350,18 +349,18 @@ void GridSolver::set_grid_volume(int nx, int ny, int nz, int conn, const uint8_t
 	const uint8_t *dv = mVolume.get();
 	if (!device_pointers) {
 		if (markers) {
-			mark.allocate(n);
-			CGP_HIP(hipMemcpyAsync(mark.get(), markers, n, hipMemcpyHostToDevice, mStream));
-			dm = mark.get();
+			mMarkers.allocate(n);
+			CGP_HIP(hipMemcpyAsync(mMarkers.get(), markers, n, hipMemcpyHostToDevice, mStream));
+			dm = mMarkers.get();
 		}
 	}
-	CGP_HIP(hipMemcpyAsync(w.get(), &weights, sizeof(weights), hipMemcpyHostToDevice, mStream));
+	CGP_HIP(hipMemcpyAsync(mWeights.get(), &weights, sizeof(weights), hipMemcpyHostToDevice, mStream));
 	const int blocks = blocks_for(n, 256, 8192);
 	if (conn == 6) {
-		hipLaunchKernelGGL(k_caps_from_volume<6>, dim3(blocks), dim3(256), 0, mStream, nx, ny, nz, dv, dm, w.get(),
+		hipLaunchKernelGGL(k_caps_from_volume<6>, dim3(blocks), dim3(256), 0, mStream, nx, ny, nz, dv, dm, mWeights.get(),
 		                   mCs.get(), mCt.get(), mCn.get());
 	} else {
-		hipLaunchKernelGGL(k_caps_from_volume<26>, dim3(blocks), dim3(256), 0, mStream, nx, ny, nz, dv, dm, w.get(),
+		hipLaunchKernelGGL(k_caps_from_volume<26>, dim3(blocks), dim3(256), 0, mStream, nx, ny, nz, dv, dm, mWeights.get(),
 		                   mCs.get(), mCt.get(), mCn.get());
 	}
 	CGP_LAUNCH_CHECK();
@@ -434,6 +433,23 @@ const InstanceDesc &GridSolver::instance(int index) const
 	return mInst[(size_t)index];
 }
 
+// Tile tables of a single grid, made by k_tile_tables: sizes and starts of the colours' groups.
+void GridSolver::size_colours(ColourSet &set, int ncolours)
+{
+	set.colours = ncolours;
+	set.size.assign(ncolours, 0);
+	for (int c = 0; c < ncolours; ++c) {
+		set.size[c] = ncolours == 2 ? face_parity_tiles(mNtx, mNty, mNtz, c) : axis_parity_tiles(mNtx, mNty, mNtz, c);
+	}
+	set.start.assign(ncolours, 0);
+	for (int c = 1; c < ncolours; ++c) {
+		set.start[c] = set.start[c - 1] + set.size[c - 1];
+	}
+	set.max_size = *std::max_element(set.size.begin(), set.size.end());
+	set.colour.allocate(((size_t)mTiles + 31) / 32 * 32, mArena);
+	set.tiles.allocate((size_t)mTiles + ncolours, mArena);
+}
+
 // Colours of every tile inside its instance: face parity (tx + ty + tz) & 1, or with corners the
 // parity per axis, so that no two tiles of a colour share a face, edge or corner.
 void GridSolver::build_colours(ColourSet &set, int ncolours, bool corners)
@@ -498,14 +514,7 @@ void GridSolver::configure_tiles(const Shape &shape)
 	mNty = mInst[0].nty;
 	mNtz = mInst[0].ntz;
 	mTiles = (int)tiles;
-	std::vector<int32_t> owner(mInst.size() > 1 ? (size_t)mTiles : 0);
-	for (size_t i = 0; i < mInst.size(); ++i) {
-		const InstanceDesc &d = mInst[i];
-		const int n = d.ntx * d.nty * d.ntz;
-		for (int t = 0; t < n && !owner.empty(); ++t) {
-			owner[(size_t)(d.tbase + t)] = (int32_t)i;
-		}
-	}
+	const bool batch = mInst.size() > 1;
 	// flag arrays padded to whole 32-byte chunks: the one-workgroup compaction reads them 16 bytes at a time
 	const int64_t padded = ((int64_t)mTiles + 31) / 32 * 32;
 	mActive.allocate(padded, mArena);
@@ -513,18 +522,37 @@ void GridSolver::configure_tiles(const Shape &shape)
 	mDirtyA.allocate(padded, mArena);
 	mDirtyB.allocate(padded, mArena);
 	mCursors.allocate(kCursorWords, mArena);
-	hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, mStream, mCursors.get(), (int64_t)kCursorWords, 0,
-	                   (const SolveControl *)nullptr, 0u);
 	mDirtyAClean = mDirtyBClean = false;  // new flag arrays
-	mAllTiles.allocate(mTiles + 1, mArena);
-	std::vector<int32_t> all(mTiles + 1);
-	for (int t = 0; t < mTiles; ++t) {
-		all[t] = t;
+	if (batch) {
+		hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, mStream, mCursors.get(), (int64_t)kCursorWords, 0,
+		                   (const SolveControl *)nullptr, 0u);
+		build_colours(mPhase, mConn == 6 ? 2 : 8, mConn != 6);
+		build_colours(mSweep, 2, false);
+	} else {
+		// one launch, no host tables and no copies
+		size_colours(mPhase, mConn == 6 ? 2 : 8);
+		size_colours(mSweep, 2);
+		TileTables out;
+		out.ntx = mNtx;
+		out.nty = mNty;
+		out.ntz = mNtz;
+		out.phase_colours = mPhase.colours;
+		out.phase_colour = mPhase.colour.get();
+		out.phase_tiles = mPhase.tiles.get();
+		out.sweep_colour = mSweep.colour.get();
+		out.sweep_tiles = mSweep.tiles.get();
+		for (int c = 0; c < mPhase.colours; ++c) {
+			out.phase_start[c] = mPhase.start[c];
+			out.phase_size[c] = mPhase.size[c];
+		}
+		for (int c = 0; c < 2; ++c) {
+			out.sweep_start[c] = mSweep.start[c];
+			out.sweep_size[c] = mSweep.size[c];
+		}
+		hipLaunchKernelGGL(k_tile_tables, dim3(blocks_for(mTiles, 256)), dim3(256), 0, mStream, out, mCursors.get(),
+		                   kCursorWords);
+		CGP_LAUNCH_CHECK();
 	}
-	all[mTiles] = mTiles;  // count slot for the all-tiles list
-	CGP_HIP(hipMemcpyAsync(mAllTiles.get(), all.data(), all.size() * sizeof(int32_t), hipMemcpyHostToDevice, mStream));
-	build_colours(mPhase, mConn == 6 ? 2 : 8, mConn != 6);
-	build_colours(mSweep, 2, false);
 	// beyond one workgroup's compaction, ordered discharge lists are laid out in class regions of
 	// the largest colour class each
 	mClassStride = mPhase.max_size;
@@ -540,7 +568,7 @@ void GridSolver::configure_tiles(const Shape &shape)
 			blocks += init_blocks(mInst[i].nx, mInst[i].ny, mInst[i].nz, mConn);
 		}
 		mInitBlocks = (int)blocks;
-		if (mInst.size() > 1) {
+		if (batch) {
 			std::vector<int32_t> owner_block((size_t)blocks);
 			for (size_t i = 0; i < mInst.size(); ++i) {
 				const int64_t end = i + 1 < mInst.size() ? first[i + 1] : blocks;
@@ -557,15 +585,20 @@ void GridSolver::configure_tiles(const Shape &shape)
 			CGP_HIP(hipStreamSynchronize(mStream));
 		}
 	}
-	if (mInst.size() > 1) {
+	if (batch) {
+		std::vector<int32_t> owner((size_t)mTiles);
+		for (size_t i = 0; i < mInst.size(); ++i) {
+			const InstanceDesc &d = mInst[i];
+			std::fill_n(owner.begin() + d.tbase, d.ntx * d.nty * d.ntz, (int32_t)i);
+		}
 		mInstDev.allocate(mInst.size(), mArena);
 		mTileInst.allocate(mTiles, mArena);
 		CGP_HIP(hipMemcpyAsync(mInstDev.get(), mInst.data(), mInst.size() * sizeof(InstanceDesc),
 		                       hipMemcpyHostToDevice, mStream));
 		CGP_HIP(hipMemcpyAsync(mTileInst.get(), owner.data(), owner.size() * sizeof(int32_t), hipMemcpyHostToDevice,
 		                       mStream));
+		CGP_HIP(hipStreamSynchronize(mStream));
 	}
-	CGP_HIP(hipStreamSynchronize(mStream));
 	mTilesReady = true;
 	mReadyShape = shape;
 }

@@ -194,12 +194,15 @@ private:
 	// Discharge phases need that no two tiles of a colour touch (2 colours for 6C, 8 for 26C); the
 	// relabel and closure sweeps only that a pass sees its face neighbours' results (face parity).
 	ColourSet mPhase, mSweep;
+	void size_colours(ColourSet &set, int ncolours);
 	void build_colours(ColourSet &set, int ncolours, bool corners);
 	int mNtx = 0, mNty = 0, mNtz = 0, mTiles = 0;
 	bool mSolved = false;
 	bool mStarted = false;  // a solve has initialised the residual state
 	int64_t mCertificate = 0;
 	DeviceBuffer<uint8_t> mVolume;  // volume of set_grid_volume
+	DeviceBuffer<uint8_t> mMarkers;
+	DeviceBuffer<cgp_volume_weights> mWeights;
 	bool mVolumeKept = false;
 	bool mStoppedEarly = false;
 	bool mLabelsExact = false;  // labels (T_min) come from an exact relabel of the final state
@@ -218,7 +221,7 @@ private:
 	DeviceBuffer<unsigned long long> mSlots, mFlow, mCounters;
 	DeviceBuffer<unsigned long long> mFlowTotal, mCounterTotal;
 	DeviceBuffer<unsigned long long> mCutSlots;  // cut capacity: kSlots slots and their sum
-	DeviceBuffer<int32_t> mStatus, mCount, mList, mAllTiles;
+	DeviceBuffer<int32_t> mStatus, mCount, mList;
 	DeviceBuffer<uint8_t> mActive, mDirtyA, mDirtyB;
 	DeviceBuffer<uint8_t> mTileWork;  // per tile: discharge work estimate from the last relabel
 	// multi-workgroup compactions: two sets of class cursors of the ordered lists, then two list

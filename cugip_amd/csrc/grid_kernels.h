@@ -464,60 +464,91 @@ __host__ __device__ constexpr int dir_index(int x, int y, int z)
 	return -1;
 }
 
+// All ones where bit d of bits is set, else 0.
+__device__ inline uint32_t spread_bit(uint32_t bits, int d) { return (uint32_t)((int32_t)(bits << (31 - d)) >> 31); }
+
+// Calls fn(k, d, label) with the label of the neighbour in direction d of own voxel k, for every
+// direction d that leaves the thread's z-column. A neighbouring column's labels are read once for
+// all own voxels beside them, and whether a direction is open or not: with a branch per direction each
+// read waited for the one before it (77 x 71 x 64, 26-connected: a solve's 48 discharge phases 2.08 ->
+// 1.59 ms, relabel passes 0.30 -> 0.17 ms; 512 x 512 x 384: relabel passes 5.77 -> 4.62 ms).
+template <typename T, typename Fn>
+__device__ inline void for_lateral_labels(const int32_t *hl, int lx, int ly, Fn &&fn)
+{
+	using D = typename T::D;
+	constexpr int kHalo = T::K == 26 ? 1 : 0;  // only diagonal directions reach the slices beyond the tile
+#pragma unroll
+	for (int y = -1; y <= 1; ++y) {
+#pragma unroll
+		for (int x = -1; x <= 1; ++x) {
+			if ((x == 0 && y == 0) || (T::K == 6 && x != 0 && y != 0)) {
+				continue;
+			}
+			int32_t nb[T::TZ + 2];
+#pragma unroll
+			for (int z = -kHalo; z < T::TZ + kHalo; ++z) {
+				nb[z + 1] = hl[T::pidx(lx + x, ly + y, z)];
+			}
+#pragma unroll
+			for (int k = 0; k < T::TZ; ++k) {
+#pragma unroll
+				for (int z = -kHalo; z <= kHalo; ++z) {
+					fn(k, dir_index<D>(x, y, z), nb[k + z + 1]);
+				}
+			}
+		}
+	}
+}
+
 // Fixpoint of h(u) = min(h(u), 1 + h(v)) over the open directions u -> v of the tile's valid
 // voxels, the halo labels fixed; hl holds the result when it returns. A round pulls the
 // directions that leave the thread's z-column from LDS and then runs the column up and down in
 // registers; the halo ends of the column never change and are read once. The fixpoint does not
-// depend on the order of the relaxations.
+// depend on the order of the relaxations. (Voxels outside the volume have no open direction.)
 template <typename T>
-__device__ inline void relax_tile(int32_t *hl, uint32_t (&open)[T::TZ], uint32_t valid, int lx, int ly)
+__device__ inline void relax_tile(int32_t *hl, const uint32_t (&open)[T::TZ], int lx, int ly)
 {
 	using D = typename T::D;
 	constexpr int kMZ = dir_index<D>(0, 0, -1), kPZ = dir_index<D>(0, 0, 1);
 	int32_t lab[T::TZ], stored[T::TZ];
+	uint32_t closed[T::TZ];
 #pragma unroll
 	for (int k = 0; k < T::TZ; ++k) {
 		lab[k] = stored[k] = hl[T::pidx(lx, ly, k)];
+		closed[k] = ~open[k];
 	}
-	const int32_t below = hl[T::pidx(lx, ly, -1)] + 1, above = hl[T::pidx(lx, ly, T::TZ)] + 1;
+	const uint32_t below = (uint32_t)hl[T::pidx(lx, ly, -1)] | spread_bit(closed[0], kMZ);
+	const uint32_t above = (uint32_t)hl[T::pidx(lx, ly, T::TZ)] | spread_bit(closed[T::TZ - 1], kPZ);
 	for (;;) {
-		// open[] is left as it is; the empty asm keeps the optimiser from hoisting per-direction
-		// lane masks out of the round loop into scalar registers
+		// the empty asm keeps the optimiser from hoisting per-direction masks out of the round loop
 #pragma unroll
 		for (int k = 0; k < T::TZ; ++k) {
-			asm volatile("" : "+v"(open[k]));
+			asm volatile("" : "+v"(closed[k]));
 		}
+		uint32_t best[T::TZ];  // lowest neighbour label over an open direction
 #pragma unroll
 		for (int k = 0; k < T::TZ; ++k) {
-			if (!((valid >> k) & 1u)) {
-				continue;
-			}
-			const int p = T::pidx(lx, ly, k);
-			int32_t best = lab[k];
+			best[k] = (uint32_t)kLabelInf;
+		}
+		for_lateral_labels<T>(hl, lx, ly, [&](int k, int d, int32_t label) {
+			const uint32_t c = (uint32_t)label | spread_bit(closed[k], d);
+			best[k] = c < best[k] ? c : best[k];
+		});
+		best[0] = below < best[0] ? below : best[0];
+		best[T::TZ - 1] = above < best[T::TZ - 1] ? above : best[T::TZ - 1];
 #pragma unroll
-			for (int d = 0; d < T::K; ++d) {
-				if ((D::dx(d) != 0 || D::dy(d) != 0) && (open[k] & (1u << d))) {
-					const int32_t nb = hl[p + T::poff(d)] + 1;
-					best = nb < best ? nb : best;
-				}
-			}
-			if (k == 0 && (open[k] & (1u << kMZ)) && below < best) {
-				best = below;
-			}
-			if (k == T::TZ - 1 && (open[k] & (1u << kPZ)) && above < best) {
-				best = above;
-			}
-			lab[k] = best;
+		for (int k = 0; k < T::TZ; ++k) {
+			lab[k] = (int32_t)best[k] + 1 < lab[k] ? (int32_t)best[k] + 1 : lab[k];
 		}
 #pragma unroll
 		for (int k = 1; k < T::TZ; ++k) {
-			if (((valid >> k) & 1u) && ((open[k] >> kMZ) & 1u) && lab[k - 1] + 1 < lab[k]) {
+			if (!((closed[k] >> kMZ) & 1u) && lab[k - 1] + 1 < lab[k]) {
 				lab[k] = lab[k - 1] + 1;
 			}
 		}
 #pragma unroll
 		for (int k = T::TZ - 2; k >= 0; --k) {
-			if (((valid >> k) & 1u) && ((open[k] >> kPZ) & 1u) && lab[k + 1] + 1 < lab[k]) {
+			if (!((closed[k] >> kPZ) & 1u) && lab[k + 1] + 1 < lab[k]) {
 				lab[k] = lab[k + 1] + 1;
 			}
 		}
@@ -533,6 +564,32 @@ __device__ inline void relax_tile(int32_t *hl, uint32_t (&open)[T::TZ], uint32_t
 		if (!__syncthreads_or(changed)) {
 			break;
 		}
+	}
+}
+
+// The open directions of the column's voxels whose neighbour is one label lower.
+template <typename T>
+__device__ inline void admissible_dirs(const int32_t *hl, const uint32_t (&open)[T::TZ], int lx, int ly,
+                                       uint32_t (&adm)[T::TZ])
+{
+	using D = typename T::D;
+	constexpr int kMZ = dir_index<D>(0, 0, -1), kPZ = dir_index<D>(0, 0, 1);
+	int32_t lab[T::TZ + 2];
+#pragma unroll
+	for (int k = -1; k <= T::TZ; ++k) {
+		lab[k + 1] = hl[T::pidx(lx, ly, k)];
+	}
+#pragma unroll
+	for (int k = 0; k < T::TZ; ++k) {
+		adm[k] = lab[k] + 1 == lab[k + 1] ? 1u << kMZ : 0u;
+		adm[k] |= lab[k + 2] + 1 == lab[k + 1] ? 1u << kPZ : 0u;
+	}
+	for_lateral_labels<T>(hl, lx, ly, [&](int k, int d, int32_t label) {
+		adm[k] |= label + 1 == lab[k + 1] ? 1u << d : 0u;
+	});
+#pragma unroll
+	for (int k = 0; k < T::TZ; ++k) {
+		adm[k] &= open[k];
 	}
 }
 
@@ -655,7 +712,7 @@ __global__ __launch_bounds__(kTX *kTY) void k_grid_bfs(GridView gv, const int32_
 		}
 	}
 	__syncthreads();
-	relax_tile<T>(hl, open, valid, lx, ly);
+	relax_tile<T>(hl, open, lx, ly);
 
 	int active = 0;
 	int top = 0, bottom = kLabelInf;
@@ -754,8 +811,16 @@ struct DirtyBits {
 	}
 };
 
+// Waves per SIMD the register allocation aims at: what the LDS of the tile allows (26-connected 32x4x2
+// tiles: 18.9 KB, 4 waves; at 3 waves, 139 VGPRs, the 512 x 512 x 384 discharge takes 13.9 instead of
+// 11.4 ms), and residual planes loaded together (all 26 in two batches instead of five: 12.0 -> 11.4 ms).
+template <int kConn, int kTZ>
+constexpr int kDischargeWaves = kConn == 6 ? 6 : kTZ == 2 ? 4 : 2;
+template <int kConn, int kTZ>
+constexpr int kDischargeLoads = kConn == 26 && kTZ == 2 ? 13 : 6;
+
 template <int kConn, int kTX, int kTY, int kTZ, typename RT>
-__global__ __launch_bounds__(kTX *kTY, 6) void k_grid_discharge(GridView gv, const int32_t *__restrict__ list,
+__global__ __launch_bounds__(kTX *kTY, (kDischargeWaves<kConn, kTZ>)) void k_grid_discharge(GridView gv, const int32_t *__restrict__ list,
                                                              const int32_t *__restrict__ count, int class_stride,
                                                              int max_iters, uint8_t *__restrict__ tile_active)
 {
@@ -822,7 +887,7 @@ __global__ __launch_bounds__(kTX *kTY, 6) void k_grid_discharge(GridView gv, con
 			el[T::vidx(lx, ly, k)] = ev[k];
 		}
 	}
-	constexpr int kGroup = 6;
+	constexpr int kGroup = kDischargeLoads<kConn, kTZ>;
 #pragma unroll
 	for (int d0 = 0; d0 < K; d0 += kGroup) {
 		int32_t rv[kGroup][T::TZ];
@@ -880,7 +945,7 @@ __global__ __launch_bounds__(kTX *kTY, 6) void k_grid_discharge(GridView gv, con
 			}
 		}
 		__syncthreads();
-		relax_tile<T>(hl, open, valid, lx, ly);
+		relax_tile<T>(hl, open, lx, ly);
 
 		// ---- per own voxel, fixed for the push sweep below: its label, its admissible directions
 		// (open, neighbour one level lower; a push never opens one, since it goes one level down)
@@ -889,23 +954,22 @@ __global__ __launch_bounds__(kTX *kTY, 6) void k_grid_discharge(GridView gv, con
 		AdmissibleDirs<K, T::TZ> adm;
 		uint32_t held = 0;
 		int top = 0;
+		{
+			uint32_t a[T::TZ];
+			admissible_dirs<T>(hl, open, lx, ly, a);
+#pragma unroll
+			for (int k = 0; k < T::TZ; ++k) {
+				adm.set(k, a[k]);
+			}
+		}
 #pragma unroll
 		for (int k = 0; k < T::TZ; ++k) {
-			const int p = T::pidx(lx, ly, k);
 			lab[k] = kLabelInf;
 			if (!(valid & (1u << k))) {
 				continue;
 			}
-			const int32_t l = hl[p];
+			const int32_t l = hl[T::pidx(lx, ly, k)];
 			lab[k] = l;
-			uint32_t a = 0;
-#pragma unroll
-			for (int d = 0; d < K; ++d) {
-				if ((open[k] & (1u << d)) && hl[p + T::poff(d)] == l - 1) {
-					a |= 1u << d;
-				}
-			}
-			adm.set(k, a);
 			if (el[T::vidx(lx, ly, k)] > 0 && l < kLabelInf) {
 				held |= 1u << k;
 				top = l > top ? l : top;

@@ -51,7 +51,8 @@ struct SolveControl {
 	int32_t active;      // active tiles at the last relabel check
 	int32_t phases;      // discharge phases run
 	int32_t max_rounds;  // round cap (kModeNotConverged beyond it)
-	int32_t pad[6];
+	int32_t discharging;  // nonzero between a relabel that found active tiles and the end of its phases
+	int32_t pad[5];
 };
 static_assert(sizeof(SolveControl) == 64, "the control block is read back as 64 bytes");
 

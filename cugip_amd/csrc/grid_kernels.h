@@ -35,9 +35,20 @@ constexpr uint32_t kStateExcess = 1u << 30;
 
 // Tile of discharge block b. A contiguous list (class_stride 0) has its length in count[0]; a list
 // in class regions (class_stride > 0) keeps class c's tiles at list + c * class_stride and their
-// number in count[c], and blocks take the classes in order. -1: no tile for this block.
-__device__ inline int discharge_tile(const int32_t *list, const int32_t *count, int class_stride, int b)
+// number in count[c], and blocks take the classes in order. class_stride < 0: the list is a phase's
+// whole colour class of -class_stride tiles, and blocks whose tile is not active have none, nor has any
+// block while count[0] is 0 (a closed gate of the device-driven solve). -1: no tile for this block.
+// The result is made wave-uniform (b is), so that tile addressing stays scalar.
+__device__ inline int discharge_tile(const int32_t *list, const int32_t *count, int class_stride, int b,
+                                     const uint8_t *active)
 {
+	if (class_stride < 0) {
+		if (b >= -class_stride || *count == 0) {
+			return -1;
+		}
+		const int tile = __builtin_amdgcn_readfirstlane(list[b]);
+		return __builtin_amdgcn_readfirstlane((int)active[tile]) ? tile : -1;
+	}
 	if (class_stride == 0) {
 		return b < *count ? list[b] : -1;
 	}
@@ -828,7 +839,7 @@ __global__ __launch_bounds__(kTX *kTY, (kDischargeWaves<kConn, kTZ>)) void k_gri
 	using D = typename T::D;
 	using Dirty = DirtyBits<kConn>;
 	constexpr int K = T::K;
-	const int tile = discharge_tile(list, count, class_stride, (int)blockIdx.x);
+	const int tile = discharge_tile(list, count, class_stride, (int)blockIdx.x, tile_active);
 	if (tile < 0) {
 		return;
 	}
@@ -1101,6 +1112,10 @@ __global__ __launch_bounds__(kTX *kTY, (kDischargeWaves<kConn, kTZ>)) void k_gri
 
 	// ---- write back what changed; pushes that left the tile go to the neighbouring voxels
 	int active = 0;
+	// (the empty asm keeps the planes' addresses of the loads from being held in registers until here:
+	// 512 x 512 x 384, 26-connected, 48 phases 11.37 -> 11.28 ms)
+	int64_t nvox = g.nvox;
+	asm volatile("" : "+s"(nvox));
 #pragma unroll
 	for (int k = 0; k < T::TZ; ++k) {
 		if (!(valid & (1u << k))) {
@@ -1130,7 +1145,7 @@ __global__ __launch_bounds__(kTX *kTY, (kDischargeWaves<kConn, kTZ>)) void k_gri
 				continue;
 			}
 			const int32_t nr = rl[d][i];
-			int32_t *plane = g.r + (int64_t)d * g.nvox;
+			int32_t *plane = g.r + (int64_t)d * nvox;
 			if (kConn != 6) {
 				const int slot = leaving_slot<T>(lx, ly, k, d);
 				if (slot >= 0) {
@@ -1140,7 +1155,7 @@ __global__ __launch_bounds__(kTX *kTY, (kDischargeWaves<kConn, kTZ>)) void k_gri
 						const int uk = k + D::dz(d);
 						const uint32_t uxy = slice_xy(g, gx + D::dx(d), gy + D::dy(d));
 						atomicAdd(&tile_at(g.e, g, oz, uk, uxy, sxy), f);
-						atomicAdd(&tile_at(g.r + (int64_t)opposite<kConn>(d) * g.nvox, g, oz, uk, uxy, sxy), f);
+						atomicAdd(&tile_at(g.r + (int64_t)opposite<kConn>(d) * nvox, g, oz, uk, uxy, sxy), f);
 						atomicOr(&tile_at(g.omask, g, oz, uk, uxy, sxy), kStateExcess | (1u << opposite<kConn>(d)));
 						marks[slot] = 1;
 					}
@@ -1357,9 +1372,20 @@ __global__ __launch_bounds__(256) void k_sum_slots(const unsigned long long *__r
 // consumed flags go back as whole 16-byte words.
 constexpr int kCompactThreads = 1024;
 // one piece per thread for up to 32768 tiles (the solver uses it with one piece; beyond, lists go
-// through the multi-workgroup passes: k_compact_tiles, or k_order_regions for the ordered
-// discharge lists, which measured faster than eight pieces a thread in one workgroup)
+// through the multi-workgroup k_compact_tiles, which measured faster than eight pieces a thread in one
+// workgroup). Discharge phases take no list up to here (kWholeColourTiles) and k_order_regions beyond.
 constexpr int kCompactBlockTiles = 32 * kCompactThreads;
+// Up to this many tiles in the grid (batch), a discharge phase launches over its whole colour class and
+// each workgroup looks at its tile's flag, and so do the sweeps of one-wave 6-connected tiles: a
+// compaction is a launch of 6 to 10 us before every pass, the workgroups without a flagged tile cost
+// less. With and without the compactions a solve takes, 26 connections (phases only): 33 x 30 x 28 1.29 ->
+// 1.13 ms, 118 x 110 x 105 2.22 -> 2.13 ms, 224 x 192 x 192 (32592 tiles) 3.62 -> 3.44 ms; 6: 33 x 30 x 28
+// 231 -> 192 us, 64 x 60 x 66 287 -> 233 us, 31 x 400 x 600 (30400 tiles) 607 -> 511 us, 224 x 192 x 192
+// 749 -> 708 us. Beyond, the idle workgroups and the order lost (heaviest first) outweigh it in the phases:
+// 256 x 256 x 256 (65536 tiles) 5.5 -> 6.3 ms and 1.11 -> 1.20 ms, 512 x 512 x 384 21.3 -> 23.4 ms and
+// 5.0 -> 5.2 ms; in the sweeps it changes nothing (256 x 256 x 256 1.10 -> 1.09 ms, 400 x 300 x 250 1.79 ->
+// 1.79 ms).
+constexpr int kWholeColourTiles = kCompactBlockTiles;
 
 __device__ inline int block_exclusive_scan_1024(int v, int *wave_sums, int &total)
 {
@@ -1493,62 +1519,13 @@ __device__ inline void compact_piece(const uint8_t *flags, const uint8_t *colour
 	}
 }
 
-// With work set (a per-tile estimate) and more than kOrderMin tiles listed (fewer all run at once),
-// the list is ordered by decreasing work class (kWorkClasses classes of work / 4, the last one
-// open-ended), in tile order within a class: the heaviest tiles start first and do not finish
-// after everyone else. The per-class counts travel packed, 16 bits a class in two 64-bit words, so
-// one workgroup scan orders all classes.
-constexpr int kOrderMin = 2048;
-
+// Work class of a tile from its per-tile estimate: kWorkClasses classes of work / 4, the heaviest
+// (open-ended) first.
 __device__ inline int work_class(int w)
 {
 	const int b = w >> 2;
 	return kWorkClasses - 1 - (b < kWorkClasses - 1 ? b : kWorkClasses - 1);
 }
-
-// Masks of the 32 tiles of a piece by work class (bit j of cm[c]: tile j is of class c), from
-// two 16-byte loads of their work bytes (one dependent load per listed tile would put a memory
-// latency on every step of the loops over the selection bits; the masks need no register array
-// indexed at run time).
-__device__ inline void class_masks(const uint8_t *work, int first, uint32_t (&cm)[kWorkClasses])
-{
-	const uint4 *p = reinterpret_cast<const uint4 *>(work + first);
-	const uint4 lo = p[0], hi = p[1];
-	const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-#pragma unroll
-	for (int c = 0; c < kWorkClasses; ++c) {
-		cm[c] = 0;
-	}
-#pragma unroll
-	for (int j = 0; j < 32; ++j) {
-		const int cls = work_class((int)((w[j >> 2] >> (8 * (j & 3))) & 0xffu));
-#pragma unroll
-		for (int c = 0; c < kWorkClasses; ++c) {
-			cm[c] |= (cls == c ? 1u : 0u) << j;
-		}
-	}
-}
-
-// The work bytes of a piece for the variant with several pieces a thread (per-class masks of every
-// piece would not fit its registers): the class of one tile at a time.
-struct PieceWork {
-	uint4 lo, hi;
-	__device__ PieceWork(const uint8_t *work, int first)
-	{
-		const uint4 *p = reinterpret_cast<const uint4 *>(work + first);
-		lo = p[0];
-		hi = p[1];
-	}
-	// work class of tile j (0 <= j < 32) of the piece
-	__device__ int cls(int j) const
-	{
-		const int d = j >> 2;
-		const uint32_t a = (d & 1) ? lo.y : lo.x, b = (d & 1) ? lo.w : lo.z;
-		const uint32_t c = (d & 1) ? hi.y : hi.x, e = (d & 1) ? hi.w : hi.z;
-		const uint32_t w = d < 4 ? ((d & 2) ? b : a) : ((d & 2) ? e : c);
-		return work_class((int)((w >> (8 * (j & 3))) & 0xffu));
-	}
-};
 
 // Exclusive scan of (lo, hi) pairs of packed counts over the workgroup; totals in tlo, thi.
 template <int kThreads = kCompactThreads>
@@ -1621,11 +1598,9 @@ __global__ __launch_bounds__(kCompactThreads) void k_compact_block(uint8_t *__re
                                                                    int32_t *__restrict__ count,
                                                                    const uint8_t *__restrict__ flags2,
                                                                    int32_t *__restrict__ count2,
-                                                                   const uint8_t *__restrict__ work,
                                                                    const SolveControl *ctl, unsigned gate)
 {
 	__shared__ int sums[2][kCompactThreads / 64];
-	__shared__ unsigned long long class_sums[kCompactThreads / 64][2];
 	if (!gate_open(ctl, gate)) {
 		// a closed gate lists nothing
 		if (threadIdx.x == 0) {
@@ -1667,8 +1642,6 @@ __global__ __launch_bounds__(kCompactThreads) void k_compact_block(uint8_t *__re
 			*count2 = total2;
 		}
 	}
-	// uniform; the packed class counts hold 16 bits, so longer lists keep tile order
-	const bool ordered = list && work && total > kOrderMin && total <= 0xffff;
 	const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
 	if (clear) {
 		if constexpr (kHold) {
@@ -1690,108 +1663,41 @@ __global__ __launch_bounds__(kCompactThreads) void k_compact_block(uint8_t *__re
 	if (!list) {
 		return;
 	}
-	if (!ordered) {
-		const int first = __shfl(pos, 0, 64), mine = pos - first, wn = sums[0][wave];
-		// (staged only with one piece a thread: with more, a thread's entries span many stage
-		// passes and it would walk its selection bits in every pass)
-		if (!kHold || wn <= kDirect) {
+	const int first = __shfl(pos, 0, 64), mine = pos - first, wn = sums[0][wave];
+	// (staged only with one piece a thread: with more, a thread's entries span many stage
+	// passes and it would walk its selection bits in every pass)
+	if (!kHold || wn <= kDirect) {
 #pragma unroll
-			for (int q = 0; q < kCompactMaxPieces; ++q) {
-				for (uint32_t m = sel[q]; m; m &= m - 1) {
-					list[pos++] = base + 32 * q + __ffs(m) - 1;
-				}
+		for (int q = 0; q < kCompactMaxPieces; ++q) {
+			for (uint32_t m = sel[q]; m; m &= m - 1) {
+				list[pos++] = base + 32 * q + __ffs(m) - 1;
 			}
-			return;
-		}
-		// A wave with many entries places them in its stage in LDS, kStage at a time, and copies
-		// them out by consecutive lanes (a thread writing its own entries straight to the list
-		// puts every lane of a store on another cache line).
-		__shared__ int stage[kCompactThreads / 64][kStage];
-		int *st = stage[wave];
-		for (int c0 = 0; c0 < wn; c0 += kStage) {
-			if (n && mine < c0 + kStage && mine + n > c0) {
-				int k = mine;
-#pragma unroll
-				for (int q = 0; q < kCompactMaxPieces; ++q) {
-					for (uint32_t m = sel[q]; m; m &= m - 1, ++k) {
-						if (k >= c0 && k < c0 + kStage) {
-							st[k - c0] = base + 32 * q + __ffs(m) - 1;
-						}
-					}
-				}
-			}
-			wave_lds_sync();
-			const int cnt = wn - c0 < kStage ? wn - c0 : kStage;
-			for (int e = lane; e < cnt; e += 64) {
-				list[first + c0 + e] = st[e];
-			}
-			wave_lds_sync();
 		}
 		return;
 	}
-	// per-class counts, 16 bits each: classes 0-3 in lo, 4-7 in hi
-	unsigned long long lo = 0, hi = 0;
+	// A wave with many entries places them in its stage in LDS, kStage at a time, and copies
+	// them out by consecutive lanes (a thread writing its own entries straight to the list
+	// puts every lane of a store on another cache line).
+	__shared__ int stage[kCompactThreads / 64][kStage];
+	int *st = stage[wave];
+	for (int c0 = 0; c0 < wn; c0 += kStage) {
+		if (n && mine < c0 + kStage && mine + n > c0) {
+			int k = mine;
 #pragma unroll
-	for (int q = 0; q < kCompactMaxPieces; ++q) {
-		if (!sel[q]) {
-			continue;
-		}
-		if constexpr (kHold) {
-			uint32_t cm[kWorkClasses];
-			class_masks(work, base + 32 * q, cm);
-#pragma unroll
-			for (int c = 0; c < kWorkClasses; ++c) {
-				const unsigned long long k = (unsigned long long)__popc(cm[c] & sel[q]) << (16 * (c & 3));
-				lo += c < 4 ? k : 0ull;
-				hi += c < 4 ? 0ull : k;
-			}
-		} else {
-			const PieceWork pw(work, base + 32 * q);
-			for (uint32_t m = sel[q]; m; m &= m - 1) {
-				const int c = pw.cls(__ffs(m) - 1);
-				const unsigned long long one = 1ull << (16 * (c & 3));
-				lo += c < 4 ? one : 0ull;
-				hi += c < 4 ? 0ull : one;
-			}
-		}
-	}
-	unsigned long long tlo = 0, thi = 0;
-	block_exclusive_scan_pair(lo, hi, class_sums, tlo, thi);
-	// class c starts after the totals of the classes before it
-	int offset[kWorkClasses];
-	int start = 0;
-#pragma unroll
-	for (int c = 0; c < kWorkClasses; ++c) {
-		const unsigned long long t = c < 4 ? tlo : thi, e = c < 4 ? lo : hi;
-		offset[c] = start + (int)((e >> (16 * (c & 3))) & 0xffffull);
-		start += (int)((t >> (16 * (c & 3))) & 0xffffull);
-	}
-#pragma unroll
-	for (int q = 0; q < kCompactMaxPieces; ++q) {
-		if (!sel[q]) {
-			continue;
-		}
-		if constexpr (kHold) {
-			uint32_t cm[kWorkClasses];
-			class_masks(work, base + 32 * q, cm);
-#pragma unroll
-			for (int c = 0; c < kWorkClasses; ++c) {
-				for (uint32_t m = cm[c] & sel[q]; m; m &= m - 1) {
-					list[offset[c]++] = base + 32 * q + __ffs(m) - 1;
-				}
-			}
-		} else {
-			const PieceWork pw(work, base + 32 * q);
-			for (uint32_t m = sel[q]; m; m &= m - 1) {
-				const int c = pw.cls(__ffs(m) - 1);
-#pragma unroll
-				for (int cc = 0; cc < kWorkClasses; ++cc) {
-					if (cc == c) {
-						list[offset[cc]++] = base + 32 * q + __ffs(m) - 1;
+			for (int q = 0; q < kCompactMaxPieces; ++q) {
+				for (uint32_t m = sel[q]; m; m &= m - 1, ++k) {
+					if (k >= c0 && k < c0 + kStage) {
+						st[k - c0] = base + 32 * q + __ffs(m) - 1;
 					}
 				}
 			}
 		}
+		wave_lds_sync();
+		const int cnt = wn - c0 < kStage ? wn - c0 : kStage;
+		for (int e = lane; e < cnt; e += 64) {
+			list[first + c0 + e] = st[e];
+		}
+		wave_lds_sync();
 	}
 }
 
@@ -1995,6 +1901,7 @@ __global__ __launch_bounds__(kCtlThreads) void k_ctl_relabel_end(SolveControl *c
 			ctl->mode = kModeNotConverged;
 		} else {
 			ctl->mode = kModeDischarge;
+			ctl->discharging = 1;
 		}
 	}
 }
@@ -2004,6 +1911,7 @@ __global__ void k_ctl_discharge_end(SolveControl *ctl, int phases)
 {
 	if (threadIdx.x == 0 && blockIdx.x == 0 && ctl->mode == kModeDischarge) {
 		ctl->phases += phases;
+		ctl->discharging = 0;
 		ctl->mode = kModeClosureNew;
 	}
 }

@@ -677,7 +677,7 @@ void GridSolver::launch_compact(const ColourSet &set, uint8_t *flags, int colour
 		launch(kCompact, 0, 0.0, [&] {
 			hipLaunchKernelGGL(k_compact_block<1>, dim3(1), dim3(kCompactThreads), 0, mStream, flags, mTiles,
 			                   set.colour.get(), colour, clear ? 1 : 0, mList.get(), mCount.get(),
-			                   (const uint8_t *)nullptr, (int32_t *)nullptr, work, ctl, gate);
+			                   (const uint8_t *)nullptr, (int32_t *)nullptr, ctl, gate);
 		});
 		mListCount = mCount.get();
 		mDischargeStride = 0;
@@ -737,7 +737,7 @@ void GridSolver::count_two(uint8_t *a, uint8_t *b, int &na, int &nb, bool defer)
 		launch(kCompact, 0, 0.0, [&] {
 			hipLaunchKernelGGL(k_compact_block<1>, dim3(1), dim3(kCompactThreads), 0, mStream, a, mTiles,
 			                   mSweep.colour.get(), -1, 0, (int32_t *)nullptr, mCount.get() + 1, (const uint8_t *)b,
-			                   mCount.get() + 2, (const uint8_t *)nullptr, (const SolveControl *)nullptr, 0u);
+			                   mCount.get() + 2, (const SolveControl *)nullptr, 0u);
 		});
 	} else {
 		// with the totals prefetched, the count's last workgroup also sums the slots
@@ -810,7 +810,9 @@ int64_t GridSolver::totals_from_readback(unsigned long long *visits)
 // until a check finds none. Tiles of one colour never touch, so each pass reads the final state
 // of the neighbours it depends on; the passes between two checks are chained on the device (each
 // reads its tile count from device memory, blocks beyond it exit), so a relabel costs one or two
-// host reads instead of one per pass. pass(list, count, grid, first) launches one pass.
+// host reads instead of one per pass. pass(list, count, grid, first) launches one pass: first c + 1, a
+// colour's first pass over all its tiles; 0, over a compacted list; -1, over the colour class whole, of
+// which the pass takes the dirty tiles (one-wave 6-connected tiles, few tiles: see kWholeColourTiles).
 // Returns the number of pass launches; `also` receives the flag count of also_count (if given)
 // at the final check.
 template <typename Pass>
@@ -822,6 +824,7 @@ int GridSolver::colour_sweeps(uint8_t *dirty, uint8_t *also_count, int &also, Pa
 	mSweepChecks = 0;
 	mSweepCycles = 0;
 	const ColourSet &cs = mSweep;
+	const bool whole = mTiles <= kWholeColourTiles && one_wave_tiles();
 	for (int c = 0; c < cs.colours; ++c) {
 		if (cs.size[c] == 0) {
 			continue;  // e.g. a grid one tile thick has no tile of the odd colours
@@ -865,8 +868,12 @@ int GridSolver::colour_sweeps(uint8_t *dirty, uint8_t *also_count, int &also, Pa
 		const int cycles = check ? kCyclesPerCheck : first_cycles;
 		for (int cycle = 0; cycle < cycles; ++cycle) {
 			for (int c = 0; c < cs.colours; ++c) {
-				launch_compact(cs, dirty, c, true);
-				pass(mList.get(), mListCount, cs.max_size, 0);
+				if (!whole) {
+					launch_compact(cs, dirty, c, true);
+					pass(mList.get(), mListCount, cs.max_size, 0);
+				} else if (cs.size[c] > 0) {
+					pass(cs.tiles.get() + cs.start[c], cs.tiles.get() + mTiles + c, cs.size[c], -1);
+				}
 				++launches;
 			}
 		}
@@ -901,7 +908,7 @@ void GridSolver::launch_bfs_pass(const int32_t *list, const int32_t *count, int 
 
 // One S_min closure pass (first: seeded from the excess). reached (may be null) is set when the
 // closure takes in a voxel with a residual sink link.
-void GridSolver::launch_closure_pass(const int32_t *list, const int32_t *count, int grid, bool first,
+void GridSolver::launch_closure_pass(const int32_t *list, const int32_t *count, int grid, int first,
                                      int32_t *reached, const SolveControl *ctl, int64_t voxels)
 {
 	GridView g = CGP_VIEW();
@@ -914,21 +921,37 @@ void GridSolver::launch_closure_pass(const int32_t *list, const int32_t *count, 
 				hipLaunchKernelGGL((k_grid_closure_wave<S::tx, S::ty, S::tz>),
 				                   dim3((grid + kPassTilesPerBlock - 1) / kPassTilesPerBlock), dim3(64 * kPassTilesPerBlock),
 				                   0, mStream, g, list,
-				                   count, first ? 1 : 0, mDirtyB.get(), reached, ctl);
+				                   count, first, mDirtyB.get(), reached, ctl);
 				return;
 			}
 			hipLaunchKernelGGL((k_grid_source_closure<S::conn, S::tx, S::ty, S::tz>), dim3(grid), dim3(S::tx * S::ty),
-			                   0, mStream, g, list, count, first ? 1 : 0, mDirtyB.get(), reached, ctl);
+			                   0, mStream, g, list, count, first, mDirtyB.get(), reached, ctl);
 		});
 	});
 }
 
+// Lists the active tiles of a colour for a discharge phase, the heaviest first (work estimates of the
+// last relabel); with few tiles in the grid a phase takes its colour class whole instead.
+void GridSolver::list_discharge_tiles(int colour, const SolveControl *ctl)
+{
+	if (mTiles > kWholeColourTiles) {
+		launch_compact(mPhase, mActive.get(), colour, false, mTileWork.get(), ctl, kGateDischarge);
+	}
+}
+
 // One discharge phase over the compacted list (every tile of one colour at most; blocks beyond
-// the count exit at once).
-void GridSolver::launch_discharge(int max_iters, bool wide)
+// the count exit at once), or over the colour class where the phase has no list.
+void GridSolver::launch_discharge(int colour, int max_iters, bool wide, const SolveControl *ctl)
 {
 	GridView g = CGP_VIEW();
-	const int blocks = mPhase.max_size;
+	const bool whole = mTiles <= kWholeColourTiles;
+	const int blocks = whole ? mPhase.size[colour] : mPhase.max_size;
+	if (blocks == 0) {
+		return;  // a grid one tile thick has no tile of some colours
+	}
+	const int32_t *list = whole ? mPhase.tiles.get() + mPhase.start[colour] : mList.get();
+	const int32_t *count = !whole ? mListCount : ctl ? &ctl->discharging : mPhase.tiles.get() + mTiles + colour;
+	const int stride = whole ? -blocks : mDischargeStride;
 	// reads and writes e, rt, h and r[K], writes the state word; one-wave 6C tiles keep the tile in
 	// registers, the others stage it in LDS with int16 residuals unless some edge's capacity pair
 	// exceeds 32767
@@ -941,16 +964,16 @@ void GridSolver::launch_discharge(int max_iters, bool wide)
 				                   dim3((blocks + kDischargeTilesPerBlock - 1) / kDischargeTilesPerBlock),
 				                   dim3(64 * kDischargeTilesPerBlock),
 				                   0, mStream, g,
-				                   mList.get(), mListCount, mDischargeStride, max_iters, mActive.get());
+				                   list, count, stride, max_iters, mActive.get());
 				return;
 			}
 			if (wide) {
 				hipLaunchKernelGGL((k_grid_discharge<S::conn, S::tx, S::ty, S::tz, int32_t>), dim3(blocks),
-				                   dim3(S::tx * S::ty), 0, mStream, g, mList.get(), mListCount, mDischargeStride,
+				                   dim3(S::tx * S::ty), 0, mStream, g, list, count, stride,
 				                   max_iters, mActive.get());
 			} else {
 				hipLaunchKernelGGL((k_grid_discharge<S::conn, S::tx, S::ty, S::tz, int16_t>), dim3(blocks),
-				                   dim3(S::tx * S::ty), 0, mStream, g, mList.get(), mListCount, mDischargeStride,
+				                   dim3(S::tx * S::ty), 0, mStream, g, list, count, stride,
 				                   max_iters, mActive.get());
 			}
 		});
@@ -980,7 +1003,7 @@ int GridSolver::run_global_relabel(int32_t threshold, cgp_stats &stats, bool def
 	stats.bfs_passes += colour_sweeps(
 	    mDirtyA.get(), mActive.get(), active,
 	    [&](const int32_t *list, const int32_t *count, int grid, int first) {
-		    launch_bfs_pass(list, count, grid, threshold, first ? grid * tile_voxels : -1, mConn == 6 ? first : 0);
+		    launch_bfs_pass(list, count, grid, threshold, first > 0 ? grid * tile_voxels : -1, mConn == 6 ? first : 0);
 	    },
 	    nullptr, defer, mRelabelCycles);
 	if (!mCheckDeferred) {
@@ -1007,9 +1030,8 @@ void GridSolver::learn_relabel_cycles(int needed)
 
 void GridSolver::run_discharge_phase(int colour, int max_iters)
 {
-	// heaviest tiles first (work estimates of the last relabel)
-	launch_compact(mPhase, mActive.get(), colour, false, mTileWork.get());
-	launch_discharge(max_iters, mWideResiduals);
+	list_discharge_tiles(colour, nullptr);
+	launch_discharge(colour, max_iters, mWideResiduals, nullptr);
 }
 
 bool GridSolver::run_source_closure(cgp_stats &stats, bool check)
@@ -1031,7 +1053,8 @@ bool GridSolver::run_source_closure(cgp_stats &stats, bool check)
 		stats.cut_passes += colour_sweeps(
 		    mDirtyB.get(), nullptr, unused,
 		    [&](const int32_t *list, const int32_t *count, int grid, int first) {
-			    launch_closure_pass(list, count, grid, first != 0, reached, nullptr, first ? grid * tile_voxels : -1);
+			    launch_closure_pass(list, count, grid, std::min(first, 1), reached, nullptr,
+			                        first > 0 ? grid * tile_voxels : -1);
 		    },
 		    check ? &hit : nullptr);
 	} catch (...) {
@@ -1134,8 +1157,8 @@ void GridSolver::capture_round_graph(int phases, int max_iters, bool wide)
 		                   (const uint8_t *)mDirtyA.get(), (const uint8_t *)mActive.get(), mTiles);
 		// discharge phases, heaviest tiles first
 		for (int p = 0; p < phases; ++p) {
-			launch_compact(mPhase, mActive.get(), p % ncolours, false, mTileWork.get(), ctl, kGateDischarge);
-			launch_discharge(max_iters, wide);
+			list_discharge_tiles(p % ncolours, ctl);
+			launch_discharge(p % ncolours, max_iters, wide, ctl);
 		}
 		hipLaunchKernelGGL(k_ctl_discharge_end, dim3(1), dim3(64), 0, mStream, ctl, phases);
 		// termination test (or the final S_min closure after a relabel found nothing active)
@@ -1145,14 +1168,14 @@ void GridSolver::capture_round_graph(int phases, int max_iters, bool wide)
 		                   kGateClosureNew);
 		for (int c = 0; c < 2; ++c) {
 			if (mSweep.size[c] > 0) {
-				launch_closure_pass(mSweep.tiles.get() + mSweep.start[c], &ctl->first[c], mSweep.size[c], true,
+				launch_closure_pass(mSweep.tiles.get() + mSweep.start[c], &ctl->first[c], mSweep.size[c], 1,
 				                    &ctl->reached, ctl, mSweep.size[c] * tile_voxels);
 			}
 		}
 		for (int cycle = 0; cycle < kGraphSweepCycles; ++cycle) {
 			for (int c = 0; c < 2; ++c) {
 				launch_compact(mSweep, mDirtyB.get(), c, true, nullptr, ctl, kGateClosure | kGateUnlessReached);
-				launch_closure_pass(mList.get(), mListCount, mSweep.max_size, false, &ctl->reached, ctl, -1);
+				launch_closure_pass(mList.get(), mListCount, mSweep.max_size, 0, &ctl->reached, ctl, -1);
 			}
 		}
 		hipLaunchKernelGGL(k_ctl_closure_end, dim3(1), dim3(kCtlThreads), 0, mStream, ctl,

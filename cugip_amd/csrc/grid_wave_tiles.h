@@ -171,7 +171,7 @@ __global__ __launch_bounds__(64 * kDischargeTilesPerBlock, 4) void k_grid_discha
 	using D = Dirs<6>;
 	constexpr int TZ = kTZ;
 	// direction bits: 0 -x, 1 -y, 2 -z, 3 +x, 4 +y, 5 +z
-	const int tile = discharge_tile(list, count, class_stride, wave_tile_index<kDischargeTilesPerBlock>());
+	const int tile = discharge_tile(list, count, class_stride, wave_tile_index<kDischargeTilesPerBlock>(), tile_active);
 	if (tile < 0) {
 		return;
 	}
@@ -468,10 +468,24 @@ __global__ __launch_bounds__(64 * kDischargeTilesPerBlock, 4) void k_grid_discha
 	}
 }
 
+// Takes a tile's dirty flag in a pass over its whole colour class (the wave's tile; face neighbours only,
+// all of the other colour, mark flags, so nothing sets this one during the pass).
+__device__ inline bool take_dirty(uint8_t *dirty, int tile)
+{
+	if (!__builtin_amdgcn_readfirstlane((int)dirty[tile])) {
+		return false;
+	}
+	if ((threadIdx.x & 63) == 0) {
+		dirty[tile] = 0;
+	}
+	return true;
+}
+
 // Global-relabel pass over a list of one-wave 6C tiles, the semantics of k_grid_bfs (labels only
 // fall; a tile whose boundary label fell below what a neighbouring voxel could use marks that
 // neighbour's tile in dirty_next; the tile's active flag and discharge work estimate are
-// refreshed; first_mode 1 / 2 as there) with the tile in registers: own labels and open directions
+// refreshed; first_mode 1 / 2 as there, -1: the list is a whole colour class, of which the dirty tiles
+// are taken) with the tile in registers: own labels and open directions
 // in the lanes, the face lanes holding the halo labels.
 template <int kTX, int kTY, int kTZ>
 __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_bfs_wave(GridView gv, const int32_t *__restrict__ list,
@@ -486,7 +500,10 @@ __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_bfs_wave(GridV
 	if (b >= *count) {
 		return;
 	}
-	const int tile = list[b];
+	const int tile = __builtin_amdgcn_readfirstlane(list[b]);
+	if (first_mode < 0 && !take_dirty(dirty_next, tile)) {
+		return;
+	}
 	int local;
 	const GridView g = instance_view(gv, tile, local);
 	int tx, ty, tz;
@@ -529,7 +546,7 @@ __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_bfs_wave(GridV
 		}
 		open[k] = o;
 		excess |= ex ? (1u << k) : 0u;
-		before[k] = (v && first_mode == 0) ? tile_at(g.h, g, oz, k, xy, sxy) : kLabelInf;
+		before[k] = (v && first_mode <= 0) ? tile_at(g.h, g, oz, k, xy, sxy) : kLabelInf;
 		lab[k] = sink_open && before[k] > 1 ? 1 : before[k];
 		hx[k] = (x_face && oz + k < g.nz) ? tile_at(g.h, g, oz, k, hxxy, sxy) : kLabelInf;
 		hy[k] = (y_face && oz + k < g.nz) ? tile_at(g.h, g, oz, k, hyxy, sxy) : kLabelInf;
@@ -552,7 +569,7 @@ __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_bfs_wave(GridV
 		active |= h;
 		top = h && nl > top ? nl : top;
 		bottom = nl < bottom ? nl : bottom;
-		if (first_mode || nl != before[k]) {
+		if (first_mode > 0 || nl != before[k]) {
 			tile_at(g.h, g, oz, k, xy, sxy) = nl;  // first passes store every label
 		}
 		if (nl != before[k]) {
@@ -593,8 +610,8 @@ __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_bfs_wave(GridV
 
 // S_min closure pass over a list of one-wave 6C tiles, the semantics of k_grid_source_closure
 // (s(u) = 1 if u holds excess or some v with s(v) = 1 has residual v -> u > 0; bits only rise;
-// first_pass seeds from the excess; the closure is pushed across the tile faces into the
-// neighbouring voxels, whose tiles are marked; `reached` is set when a voxel with a residual sink
+// first_pass 1 seeds from the excess, -1: the list is a whole colour class, of which the dirty tiles are
+// taken; the closure is pushed across the tile faces into the neighbouring voxels, whose tiles are marked; `reached` is set when a voxel with a residual sink
 // link joins) with the tile in registers: a lane's s bits and open directions travel together to
 // its x and y neighbour lanes, the column is swept up and down in registers.
 template <int kTX, int kTY, int kTZ>
@@ -610,7 +627,10 @@ __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_closure_wave(G
 	if (b >= *count || !gate_open(ctl, kGateClosure | kGateUnlessReached)) {
 		return;
 	}
-	const int tile = list[b];
+	const int tile = __builtin_amdgcn_readfirstlane(list[b]);
+	if (first_pass < 0 && !take_dirty(dirty_next, tile)) {
+		return;
+	}
 	int local;
 	const GridView g = instance_view(gv, tile, local);
 	int tx, ty, tz;
@@ -632,7 +652,7 @@ __global__ __launch_bounds__(64 * kPassTilesPerBlock) void k_grid_closure_wave(G
 		open[k] = st & 63u;
 		before |= b ? (1u << k) : 0u;
 		sink |= (st & kStateSink) ? (1u << k) : 0u;
-		sbits |= (b || (first_pass && (st & kStateExcess))) ? (1u << k) : 0u;
+		sbits |= (b || (first_pass > 0 && (st & kStateExcess))) ? (1u << k) : 0u;
 	}
 	// fixpoint inside the tile: a lane's s bit with its open directions (bit 6 and bits 0-5) go to
 	// the x and y neighbour lanes of the same z-level

@@ -124,9 +124,12 @@ private:
 	                    const uint8_t *work = nullptr, const SolveControl *ctl = nullptr, unsigned gate = 0);
 	void launch_bfs_pass(const int32_t *list, const int32_t *count, int grid, int32_t threshold, int64_t voxels,
 	                     int first_mode);
-	void launch_closure_pass(const int32_t *list, const int32_t *count, int grid, bool first, int32_t *reached,
+	void launch_closure_pass(const int32_t *list, const int32_t *count, int grid, int first, int32_t *reached,
 	                         const SolveControl *ctl, int64_t voxels);
-	void launch_discharge(int max_iters, bool wide);
+	void list_discharge_tiles(int colour, const SolveControl *ctl);
+	// 6-connected tiles kept in the registers of one wave (grid_wave_tiles.h)
+	bool one_wave_tiles() const { return mConn == 6 && mShape.tx * mShape.ty == 64; }
+	void launch_discharge(int colour, int max_iters, bool wide, const SolveControl *ctl);
 	void count_two(uint8_t *a, uint8_t *b, int &na, int &nb, bool defer = false);
 	void count_two_wait(int &na, int &nb, bool has_b);
 	const int32_t *deferred_counts() const;

@@ -235,9 +235,18 @@ __global__ __launch_bounds__(256) void k_conv(int nx, int ny, int nz, const uint
 	}
 }
 
-// Forward layer, marching along z: workgroup (bx, by, bz) computes zbricks (z_bricks below) consecutive 16 x 4 x 4 output bricks in z. The input planes stay in an LDS ring of 8 z-planes
-// (one plane per 4-channel group as in k_conv), so each brick stages only the 4 planes it adds
-// instead of its whole 6-plane halo box. Same arithmetic and output as k_conv<CIN, false, HEAD>.
+// Forward layer, marching along z: workgroup (bx, by, bz) computes zbricks (z_bricks below) consecutive
+// 16 x 4 x 4 output bricks in z. The input planes stay in an LDS ring of 8 z-planes (one plane per
+// 4-channel group as in k_conv), so each brick stages only the 4 planes it adds instead of its whole
+// 6-plane halo box. Same arithmetic and output as k_conv<CIN, false, HEAD>.
+//
+// What bounds it: 64 bytes of traffic a voxel (82 us of the 121 at 200 x 190 x 157) and the 27 products of
+// 16 voxels (half of the 43 us at 131 x 125 x 119). So the planes of the next brick are loaded into
+// registers under this brick's products (loaded and stored a plane at a time between two barriers, each
+// plane cost a memory latency: 60 -> 49 us a 16-channel layer at 131 x 125 x 119, 194 -> 157 us at 200 x 190
+// x 157), and a wave takes the four rows of its slice together: 54 instead of 108 LDS reads and four
+// independent sums (49 -> 43 and 157 -> 121 us; without the prefetch the rows gave nothing, 60 -> 65 us).
+// The registers fit four waves per SIMD (three, the head layer takes 51 instead of 47 us).
 constexpr int kZSlots = 8;
 
 // Per-thread staging map of one input z-plane of the brick box (18 x 6 voxels, CIN / 4 channel
@@ -271,26 +280,34 @@ struct PlaneMap {
 		}
 	}
 
-	__device__ void stage(uint16_t *lds, const uint16_t *__restrict__ in, int nx, int ny, int nz, int z) const
+	// the entries of plane z, zero outside the volume
+	__device__ void load(uint2 (&val)[kIters], const uint16_t *__restrict__ in, int nx, int ny, int nz, int z) const
 	{
 		const bool zin = z >= 0 && z < nz;
 		const uint16_t *slice = in + (zin ? (int64_t)z * nx * ny * CIN : 0);
+#pragma unroll
+		for (int i = 0; i < kIters; ++i) {
+			val[i] = make_uint2(0u, 0u);
+			if (zin && ((inside >> i) & 1u)) {
+				val[i] = *reinterpret_cast<const uint2 *>(slice + goff[i]);
+			}
+		}
+	}
+
+	__device__ void store(uint16_t *lds, const uint2 (&val)[kIters], int z) const
+	{
 		const uint32_t soff = ((uint32_t)(z + kZSlots) & (uint32_t)(kZSlots - 1)) * PL * 4;
 #pragma unroll
 		for (int i = 0; i < kIters; ++i) {
 			if ((exists >> i) & 1u) {
-				uint2 val = make_uint2(0u, 0u);
-				if (zin && ((inside >> i) & 1u)) {
-					val = *reinterpret_cast<const uint2 *>(slice + goff[i]);
-				}
-				*reinterpret_cast<uint2 *>(lds + loff[i] + soff) = val;
+				*reinterpret_cast<uint2 *>(lds + loff[i] + soff) = val[i];
 			}
 		}
 	}
 };
 
 template <int CIN, bool HEAD>
-__global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, const uint16_t *__restrict__ in,
+__global__ __launch_bounds__(256, 4) void k_conv_fwd_z(int nx, int ny, int nz, const uint16_t *__restrict__ in,
                                                    const uint16_t *__restrict__ pack, const float *__restrict__ bias,
                                                    uint16_t *__restrict__ out, const float *__restrict__ head,
                                                    float *__restrict__ logits, int zbricks)
@@ -317,10 +334,18 @@ __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, cons
 	}
 	PlaneMap<CIN> map;
 	map.init(nx, ny, bx, by);
-#pragma unroll 1
-	for (int p = -1; p <= BZ; ++p) {
-		map.stage(lds, in, nx, ny, nz, bz0 + p);
+	{
+		uint2 box[HZ][PlaneMap<CIN>::kIters];
+#pragma unroll
+		for (int p = 0; p < HZ; ++p) {
+			map.load(box[p], in, nx, ny, nz, bz0 + p - 1);
+		}
+#pragma unroll
+		for (int p = 0; p < HZ; ++p) {
+			map.store(lds, box[p], bz0 + p - 1);
+		}
 	}
+	__syncthreads();
 	// the lane's LDS base: its channel group's planes, its voxel column (x + 1 for the halo)
 	const uint32_t lbase = (uint32_t)((((CIN == 16 ? grp : 0) * kZSlots * PL) + col + 1) * 4);
 	const int lz = wave;
@@ -329,40 +354,66 @@ __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, cons
 		if (bz >= nz) {
 			break;  // uniform across the workgroup
 		}
-		if (zb > 0) {
-			__syncthreads();  // the previous brick's reads of the slots about to be refilled are done
-#pragma unroll 1
-			for (int p = 1; p <= BZ; ++p) {
-				map.stage(lds, in, nx, ny, nz, bz + p);
+		// the planes the next brick adds are loaded under this brick's products
+		const bool more = zb + 1 < zbricks && bz + BZ < nz;  // uniform across the workgroup
+		uint2 ahead[BZ][PlaneMap<CIN>::kIters];
+		if (more) {
+#pragma unroll
+			for (int p = 0; p < BZ; ++p) {
+				map.load(ahead[p], in, nx, ny, nz, bz + BZ + 1 + p);
 			}
 		}
-		__syncthreads();
 		// ring slot offsets of the planes z - 1, z, z + 1 of this wave's output slice
 		uint32_t sdz[3];
 #pragma unroll
 		for (int d = 0; d < 3; ++d) {
 			sdz[d] = ((uint32_t)(bz + lz + d - 1 + kZSlots) & (uint32_t)(kZSlots - 1)) * PL * 4;
 		}
-#pragma unroll 1
+		float4_t acc[BY];
+#pragma unroll
 		for (int ly = 0; ly < BY; ++ly) {
-			float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+			acc[ly] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+		}
+		if constexpr (CIN == 16) {
+			// Each row of the brick box is read once for the (up to three) output rows it touches; every
+			// output row still adds its taps in order 0 .. 26.
+#pragma unroll
+			for (int dz = 0; dz < 3; ++dz) {
+#pragma unroll
+				for (int hy = 0; hy < HY; ++hy) {
+					short4_t b[3];  // compile-time offsets: the reads take immediate offsets
+#pragma unroll
+					for (int dx = 0; dx < 3; ++dx) {
+						b[dx] = *reinterpret_cast<const short4_t *>(lds + lbase + sdz[dz] + (hy * HX + dx - 1) * 4);
+					}
+#pragma unroll
+					for (int dx = 0; dx < 3; ++dx) {
+#pragma unroll
+						for (int ly = 0; ly < BY; ++ly) {
+							const int dy = hy - ly;
+							if (dy >= 0 && dy < 3) {
+								acc[ly] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[(dz * 3 + dy) * 3 + dx], b[dx], acc[ly], 0,
+								                                                    0, 0);
+							}
+						}
+					}
+				}
+			}
+		} else {
 #pragma unroll
 			for (int m = 0; m < NM; ++m) {
-				short4_t b;
-				if constexpr (CIN == 16) {
-					const int t = m;  // compile-time offsets: the reads take immediate offsets
-					const uint32_t off = sdz[tap_dz(t) + 1] +
-					                     (uint32_t)((((ly + 1 + tap_dy(t)) * HX) + tap_dx(t)) * 4);
-					b = *reinterpret_cast<const short4_t *>(lds + lbase + off);
-				} else {
-					int t = 4 * m + grp;
-					t = t < kCnnTaps ? t : kCnnTaps - 1;  // padded taps have zero weights
-					const uint32_t off = sdz[tap_dz(t) + 1] +
-					                     (uint32_t)((((ly + 1 + tap_dy(t)) * HX) + tap_dx(t)) * 4);
-					b = *reinterpret_cast<const short4_t *>(lds + lbase + off);
+				int t = 4 * m + grp;
+				t = t < kCnnTaps ? t : kCnnTaps - 1;  // padded taps have zero weights
+				const uint32_t off = sdz[tap_dz(t) + 1] + (uint32_t)((((1 + tap_dy(t)) * HX) + tap_dx(t)) * 4);
+#pragma unroll
+				for (int ly = 0; ly < BY; ++ly) {
+					const short4_t b = *reinterpret_cast<const short4_t *>(lds + lbase + off + ly * HX * 4);
+					acc[ly] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b, acc[ly], 0, 0, 0);
 				}
-				acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b, acc, 0, 0, 0);
 			}
+		}
+#pragma unroll
+		for (int ly = 0; ly < BY; ++ly) {
 			const int x = bx + col, y = by + ly, z = bz + lz;
 			const bool valid = x < nx && y < ny && z < nz;
 			const int64_t v = ((int64_t)z * ny + y) * nx + x;
@@ -371,7 +422,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, cons
 			float head_part = 0.0f;
 #pragma unroll
 			for (int j = 0; j < 4; ++j) {
-				float val = acc[j] + bias4[j];
+				float val = acc[ly][j] + bias4[j];
 				val = val > 0.0f ? val : 0.0f;
 				r[j] = f2bf(val);
 				if (HEAD) {
@@ -392,6 +443,14 @@ __global__ __launch_bounds__(256) void k_conv_fwd_z(int nx, int ny, int nz, cons
 					logits[v] = head_part + head[kCnnChannels];
 				}
 			}
+		}
+		if (more) {
+			__syncthreads();  // the reads of the slots about to be refilled are done
+#pragma unroll
+			for (int p = 0; p < BZ; ++p) {
+				map.store(lds, ahead[p], bz + BZ + 1 + p);
+			}
+			__syncthreads();
 		}
 	}
 }
@@ -773,10 +832,10 @@ __global__ __launch_bounds__(256) void k_sigmoid(int64_t n, const float *__restr
 }
 
 // Bricks a workgroup of the forward layers marches: long marches stage fewer halo planes, short ones
-// fill the chip. Five workgroups fit a CU (LDS), so 8 bricks need some 2500 workgroups to keep the last
+// fill the chip. Four workgroups fit a CU (registers), so 8 bricks need some 2500 workgroups to keep the last
 // ones from running alone, and below 512 half the CUs idle. 16 -> 16 layer with 8 / 6 / 4 / 2 / 1 bricks:
-// 131 x 125 x 119 voxels 59 / 71 / 59 / 66 / 72 us (with the head 81 / 78 / 70 / 76 / 85),
-// 98 x 96 x 91: 44 / 37 / 31 / 32 / 35 us.
+// 131 x 125 x 119 voxels 47 / 46 / 43 / 45 / 49 us (with the head 51 / 50 / 47 / 50 / 54),
+// 98 x 96 x 91: 27 / 25 / 24 / 24 / 26 us.
 int z_bricks(int nx, int ny, int nz)
 {
 	const int64_t columns = (int64_t)((nx + BX - 1) / BX) * ((ny + BY - 1) / BY);

@@ -1,15 +1,13 @@
 // Learned cut proposal on the matrix cores: 3D convolutions as implicit GEMMs with
 // v_mfma_f32_16x16x16_bf16 (BF16 operands, FP32 accumulation), their backward passes, Adam.
 //
-// One workgroup (4 waves) owns an output brick of 16 x 4 x 4 voxels and stages its input brick
-// with a one-voxel halo (18 x 6 x 6 voxels, BF16, one LDS plane per group of 4 channels) in LDS. A
-// wave computes one row
-// of 16 voxels at a time as D = A x B per tap: A = the 16 x 16 weight block of the tap (held in
-// registers for all taps), B = the 16 channels of the 16 voxels shifted by the tap offset (from
-// LDS), D = 16 output channels x 16 voxels. In the MFMA's lane layout, lane l holds voxel l % 16
-// and channels 4 * (l / 16) .. + 3 of D, so each lane stores 8 contiguous bytes. Inference
-// (k_conv_fwd_z) walks several bricks along z per workgroup and keeps the input planes in an LDS
-// ring, staging only the planes each brick adds.
+// One workgroup (4 waves) walks output bricks of 16 x 4 x 4 voxels along z and keeps the input planes
+// with a one-voxel halo (18 x 6 voxels, BF16, one LDS plane per group of 4 channels) in an LDS ring,
+// staging only the planes each brick adds (k_conv_z). A wave computes the four rows of 16 voxels of its
+// z-slice as D = A x B per tap: A = the 16 x 16 weight block of the tap (held in registers for all taps),
+// B = the 16 channels of the 16 voxels shifted by the tap offset (from LDS), D = 16 output channels x 16
+// voxels. In the MFMA's lane layout, lane l holds voxel l % 16 and channels 4 * (l / 16) .. + 3 of D, so
+// each lane stores 8 contiguous bytes.
 #include <cmath>
 #include <cstring>
 
@@ -115,130 +113,16 @@ __global__ __launch_bounds__(256) void k_cnn_input(int64_t n, const uint8_t *__r
 	}
 }
 
-// Stage the input brick with its halo as one plane per group of 4 channels (8 bytes a voxel), so
-// that the 16 lanes of an MFMA B fragment, which read one channel group of 16 consecutive voxels,
-// read 128 contiguous bytes (channel-last, their 8-byte reads would stride 32 bytes and collide in
-// the LDS banks). Zero outside the volume.
-template <int CIN>
-__device__ inline void stage_brick_planar(uint16_t *lds, const uint16_t *__restrict__ in, int nx, int ny, int nz,
-                                          int bx, int by, int bz)
-{
-	constexpr int kParts = CIN / 4;
-	for (int e = threadIdx.x; e < HV * kParts; e += blockDim.x) {
-		const int hv = e / kParts, part = e % kParts;
-		const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-		const int x = bx + hx - 1, y = by + hy - 1, z = bz + hz - 1;
-		uint2 val = make_uint2(0u, 0u);
-		if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) {
-			const int64_t v = ((int64_t)z * ny + y) * nx + x;
-			val = *reinterpret_cast<const uint2 *>(in + v * CIN + part * 4);
-		}
-		*reinterpret_cast<uint2 *>(lds + (part * HV + hv) * 4) = val;
-	}
-}
-
 // Convolution layer. Forward (BWD false): out = ReLU(conv(in, W) + b) in bf16; with HEAD, also
 // logit = w_head . out + b_head (the sigmoid head fused into the last layer). Backward data (BWD
 // true, CIN 16): out = conv^T(g, W) masked by (mask_act > 0), the gradient at the pre-activation
 // of the layer below.
-template <int CIN, bool BWD, bool HEAD>
-__global__ __launch_bounds__(256) void k_conv(int nx, int ny, int nz, const uint16_t *__restrict__ in,
-                                             const uint16_t *__restrict__ pack, const float *__restrict__ bias,
-                                             const uint16_t *__restrict__ mask_act, uint16_t *__restrict__ out,
-                                             const float *__restrict__ head, float *__restrict__ logits)
-{
-	__shared__ __attribute__((aligned(16))) uint16_t lds[HV * CIN];
-	const int bx = blockIdx.x * BX, by = blockIdx.y * BY, bz = blockIdx.z * BZ;
-	stage_brick_planar<CIN>(lds, in, nx, ny, nz, bx, by, bz);
-	constexpr int NM = CIN == 16 ? 27 : 7;
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	const int col = lane & 15, grp = lane >> 4;
-	short4_t a[NM];
-#pragma unroll
-	for (int m = 0; m < NM; ++m) {
-		a[m] = *reinterpret_cast<const short4_t *>(pack + (m * 64 + lane) * 4);
-	}
-	float bias4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-	float hw4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-	if (!BWD) {
-#pragma unroll
-		for (int j = 0; j < 4; ++j) {
-			bias4[j] = bias[4 * grp + j];
-			if (HEAD) {
-				hw4[j] = head[4 * grp + j];
-			}
-		}
-	}
-	__syncthreads();
-#pragma unroll 1
-	for (int i = 0; i < 4; ++i) {
-		const int row = wave * 4 + i;
-		const int ly = row % BY, lz = row / BY;
-		float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-		for (int m = 0; m < NM; ++m) {
-			int t;
-			int c0;
-			if (CIN == 16) {
-				t = BWD ? kCnnTaps - 1 - m : m;  // backward reads g at u - off(t) = u + off(26 - t)
-				c0 = 4 * grp;
-			} else {
-				t = 4 * m + grp;
-				t = t < kCnnTaps ? t : kCnnTaps - 1;  // padded taps have zero weights
-				c0 = 0;
-			}
-			const int hv = ((lz + 1 + tap_dz(t)) * HY + (ly + 1 + tap_dy(t))) * HX + (col + 1 + tap_dx(t));
-			const short4_t b = *reinterpret_cast<const short4_t *>(lds + ((c0 / 4) * HV + hv) * 4);
-			acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b, acc, 0, 0, 0);
-		}
-		const int x = bx + col, y = by + ly, z = bz + lz;
-		const bool valid = x < nx && y < ny && z < nz;
-		const int64_t v = ((int64_t)z * ny + y) * nx + x;
-		ushort4 q;
-		uint16_t r[4];
-		float head_part = 0.0f;
-#pragma unroll
-		for (int j = 0; j < 4; ++j) {
-			float val = acc[j];
-			if (!BWD) {
-				val += bias4[j];
-				val = val > 0.0f ? val : 0.0f;
-				r[j] = f2bf(val);
-				if (HEAD) {
-					head_part += hw4[j] * bf2f(r[j]);
-				}
-			} else {
-				r[j] = 0;
-			}
-		}
-		if (BWD && valid) {
-			const ushort4 mk = *reinterpret_cast<const ushort4 *>(mask_act + v * 16 + 4 * grp);
-			r[0] = mk.x ? f2bf(acc[0]) : 0;
-			r[1] = mk.y ? f2bf(acc[1]) : 0;
-			r[2] = mk.z ? f2bf(acc[2]) : 0;
-			r[3] = mk.w ? f2bf(acc[3]) : 0;
-		}
-		q.x = r[0];
-		q.y = r[1];
-		q.z = r[2];
-		q.w = r[3];
-		if (HEAD) {
-			head_part += __shfl_xor(head_part, 16, 64);
-			head_part += __shfl_xor(head_part, 32, 64);
-		}
-		if (valid) {
-			*reinterpret_cast<ushort4 *>(out + v * 16 + 4 * grp) = q;
-			if (HEAD && grp == 0) {
-				logits[v] = head_part + head[kCnnChannels];
-			}
-		}
-	}
-}
-
-// Forward layer, marching along z: workgroup (bx, by, bz) computes zbricks (z_bricks below) consecutive
-// 16 x 4 x 4 output bricks in z. The input planes stay in an LDS ring of 8 z-planes (one plane per
-// 4-channel group as in k_conv), so each brick stages only the 4 planes it adds instead of its whole
-// 6-plane halo box. Same arithmetic and output as k_conv<CIN, false, HEAD>.
+//
+// It marches along z: workgroup (bx, by, bz) computes zbricks (z_bricks below) consecutive
+// 16 x 4 x 4 output bricks in z. The input planes stay in an LDS ring of 8 z-planes, one plane per group of
+// 4 channels: a wave's 16 lanes of a channel group read 128 contiguous bytes (channel-last, their 8-byte
+// reads would stride 32 bytes and collide in the LDS banks). Each brick stages only the 4 planes it adds
+// instead of its whole 6-plane halo box.
 //
 // What bounds it: 64 bytes of traffic a voxel (82 us of the 121 at 200 x 190 x 157) and the 27 products of
 // 16 voxels (half of the 43 us at 131 x 125 x 119). So the planes of the next brick are loaded into
@@ -247,6 +131,8 @@ __global__ __launch_bounds__(256) void k_conv(int nx, int ny, int nz, const uint
 // x 157), and a wave takes the four rows of its slice together: 54 instead of 108 LDS reads and four
 // independent sums (49 -> 43 and 157 -> 121 us; without the prefetch the rows gave nothing, 60 -> 65 us).
 // The registers fit four waves per SIMD (three, the head layer takes 51 instead of 47 us).
+// Backward data as bricks that stage their whole halo box took 36 instead of 28 us a layer at 98 x 96 x 91
+// and 244 instead of 162 us at 200 x 190 x 157.
 constexpr int kZSlots = 8;
 
 // Per-thread staging map of one input z-plane of the brick box (18 x 6 voxels, CIN / 4 channel
@@ -306,9 +192,10 @@ struct PlaneMap {
 	}
 };
 
-template <int CIN, bool HEAD>
-__global__ __launch_bounds__(256, 4) void k_conv_fwd_z(int nx, int ny, int nz, const uint16_t *__restrict__ in,
+template <int CIN, bool BWD, bool HEAD>
+__global__ __launch_bounds__(256, 4) void k_conv_z(int nx, int ny, int nz, const uint16_t *__restrict__ in,
                                                    const uint16_t *__restrict__ pack, const float *__restrict__ bias,
+                                                  const uint16_t *__restrict__ mask_act,
                                                    uint16_t *__restrict__ out, const float *__restrict__ head,
                                                    float *__restrict__ logits, int zbricks)
 {
@@ -324,12 +211,14 @@ __global__ __launch_bounds__(256, 4) void k_conv_fwd_z(int nx, int ny, int nz, c
 	for (int m = 0; m < NM; ++m) {
 		a[m] = *reinterpret_cast<const short4_t *>(pack + (m * 64 + lane) * 4);
 	}
-	float bias4[4], hw4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+	float bias4[4] = {0.0f, 0.0f, 0.0f, 0.0f}, hw4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+	if (!BWD) {
 #pragma unroll
-	for (int j = 0; j < 4; ++j) {
-		bias4[j] = bias[4 * grp + j];
-		if (HEAD) {
-			hw4[j] = head[4 * grp + j];
+		for (int j = 0; j < 4; ++j) {
+			bias4[j] = bias[4 * grp + j];
+			if (HEAD) {
+				hw4[j] = head[4 * grp + j];
+			}
 		}
 	}
 	PlaneMap<CIN> map;
@@ -369,6 +258,17 @@ __global__ __launch_bounds__(256, 4) void k_conv_fwd_z(int nx, int ny, int nz, c
 		for (int d = 0; d < 3; ++d) {
 			sdz[d] = ((uint32_t)(bz + lz + d - 1 + kZSlots) & (uint32_t)(kZSlots - 1)) * PL * 4;
 		}
+		ushort4 mask[BY];
+		if (BWD) {
+#pragma unroll
+			for (int ly = 0; ly < BY; ++ly) {
+				const int x = bx + col, y = by + ly, z = bz + lz;
+				mask[ly] = make_ushort4(0, 0, 0, 0);
+				if (x < nx && y < ny && z < nz) {
+					mask[ly] = *reinterpret_cast<const ushort4 *>(mask_act + (((int64_t)z * ny + y) * nx + x) * 16 + 4 * grp);
+				}
+			}
+		}
 		float4_t acc[BY];
 #pragma unroll
 		for (int ly = 0; ly < BY; ++ly) {
@@ -376,24 +276,28 @@ __global__ __launch_bounds__(256, 4) void k_conv_fwd_z(int nx, int ny, int nz, c
 		}
 		if constexpr (CIN == 16) {
 			// Each row of the brick box is read once for the (up to three) output rows it touches; every
-			// output row still adds its taps in order 0 .. 26.
+			// output row still adds its weight blocks in order 0 .. 26 (backward they are packed from the last
+			// tap to the first: it reads g at u - off(t) = u + off(26 - t)).
 #pragma unroll
-			for (int dz = 0; dz < 3; ++dz) {
+			for (int iz = 0; iz < 3; ++iz) {
+				const int dz = BWD ? 2 - iz : iz;
 #pragma unroll
-				for (int hy = 0; hy < HY; ++hy) {
+				for (int ih = 0; ih < HY; ++ih) {
+					const int hy = BWD ? HY - 1 - ih : ih;
 					short4_t b[3];  // compile-time offsets: the reads take immediate offsets
 #pragma unroll
 					for (int dx = 0; dx < 3; ++dx) {
 						b[dx] = *reinterpret_cast<const short4_t *>(lds + lbase + sdz[dz] + (hy * HX + dx - 1) * 4);
 					}
 #pragma unroll
-					for (int dx = 0; dx < 3; ++dx) {
+					for (int ix = 0; ix < 3; ++ix) {
+						const int dx = BWD ? 2 - ix : ix;
 #pragma unroll
 						for (int ly = 0; ly < BY; ++ly) {
 							const int dy = hy - ly;
 							if (dy >= 0 && dy < 3) {
-								acc[ly] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[(dz * 3 + dy) * 3 + dx], b[dx], acc[ly], 0,
-								                                                    0, 0);
+								const int t = (dz * 3 + dy) * 3 + dx, m = BWD ? kCnnTaps - 1 - t : t;
+								acc[ly] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b[dx], acc[ly], 0, 0, 0);
 							}
 						}
 					}
@@ -422,12 +326,22 @@ __global__ __launch_bounds__(256, 4) void k_conv_fwd_z(int nx, int ny, int nz, c
 			float head_part = 0.0f;
 #pragma unroll
 			for (int j = 0; j < 4; ++j) {
-				float val = acc[ly][j] + bias4[j];
-				val = val > 0.0f ? val : 0.0f;
-				r[j] = f2bf(val);
-				if (HEAD) {
-					head_part += hw4[j] * bf2f(r[j]);
+				r[j] = 0;
+				if (!BWD) {
+					float val = acc[ly][j] + bias4[j];
+					val = val > 0.0f ? val : 0.0f;
+					r[j] = f2bf(val);
+					if (HEAD) {
+						head_part += hw4[j] * bf2f(r[j]);
+					}
 				}
+			}
+			if (BWD && valid) {
+				const ushort4 mk = mask[ly];
+				r[0] = mk.x ? f2bf(acc[ly][0]) : 0;
+				r[1] = mk.y ? f2bf(acc[ly][1]) : 0;
+				r[2] = mk.z ? f2bf(acc[ly][2]) : 0;
+				r[3] = mk.w ? f2bf(acc[ly][3]) : 0;
 			}
 			q.x = r[0];
 			q.y = r[1];
@@ -941,16 +855,17 @@ void CnnModel::forward(GridSolver &grid, const uint8_t *volume, bool device_volu
 	const int zbricks = z_bricks(mNx, mNy, mNz);
 	const dim3 gridz((mNx + BX - 1) / BX, (mNy + BY - 1) / BY, (mNz + BZ * zbricks - 1) / (BZ * zbricks));
 	const float *p = mParams.get();
-	hipLaunchKernelGGL((k_conv_fwd_z<4, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mX0.get(),
-	                   mPackFwd.get() + pack_fwd_off(0), p + off_b(0), mAct[0].get(), (const float *)nullptr,
+	hipLaunchKernelGGL((k_conv_z<4, false, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mX0.get(),
+	                   mPackFwd.get() + pack_fwd_off(0), p + off_b(0), (const uint16_t *)nullptr, mAct[0].get(), (const float *)nullptr,
 	                   (float *)nullptr, zbricks);
 	for (int layer = 1; layer <= 2; ++layer) {
-		hipLaunchKernelGGL((k_conv_fwd_z<16, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz,
+		hipLaunchKernelGGL((k_conv_z<16, false, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz,
 		                   mAct[layer - 1].get(), mPackFwd.get() + pack_fwd_off(layer), p + off_b(layer),
-		                   mAct[layer].get(), (const float *)nullptr, (float *)nullptr, zbricks);
+		                   (const uint16_t *)nullptr, mAct[layer].get(), (const float *)nullptr, (float *)nullptr, zbricks);
 	}
-	hipLaunchKernelGGL((k_conv_fwd_z<16, true>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mAct[2].get(),
-	                   mPackFwd.get() + pack_fwd_off(3), p + off_b(3), mAct[3].get(), p + kOffHeadW, mLogit.get(), zbricks);
+	hipLaunchKernelGGL((k_conv_z<16, false, true>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mAct[2].get(),
+	                   mPackFwd.get() + pack_fwd_off(3), p + off_b(3), (const uint16_t *)nullptr, mAct[3].get(),
+	                   p + kOffHeadW, mLogit.get(), zbricks);
 	hipLaunchKernelGGL(k_threshold, dim3(blocks_of(mVox)), dim3(256), 0, mStream, mVox, mLogit.get(), mSide.get());
 	CGP_LAUNCH_CHECK();
 	if (wait) {
@@ -1000,7 +915,8 @@ void CnnModel::run_backward(GridSolver &grid, double &loss)
 	hipLaunchKernelGGL(k_sum_scalars, dim3(1), dim3(256), 0, mStream, mScalars.get(), head_blocks,
 	                   mGrad.get() + kOffHeadB);
 	reduce(head_blocks, 16, mGrad.get() + kOffHeadW);
-	const dim3 grid3(nbx, nby, nbz);
+	const int zbricks = z_bricks(mNx, mNy, mNz);
+	const dim3 gridz(nbx, nby, (nbz + zbricks - 1) / zbricks);
 	int cur = 0;
 	for (int layer = 3; layer >= 1; --layer) {
 		// weight gradient of `layer` (input: activation of layer - 1, gradient at its pre-activation in mG[cur])
@@ -1008,9 +924,9 @@ void CnnModel::run_backward(GridSolver &grid, double &loss)
 		                   mAct[layer - 1].get(), mG[cur].get(), mPartials.get());
 		reduce(wg_blocks, per16, mGrad.get() + off_w(layer));
 		// gradient at the pre-activation of layer - 1
-		hipLaunchKernelGGL((k_conv<16, true, false>), grid3, dim3(256), 0, mStream, mNx, mNy, mNz, mG[cur].get(),
+		hipLaunchKernelGGL((k_conv_z<16, true, false>), gridz, dim3(256), 0, mStream, mNx, mNy, mNz, mG[cur].get(),
 		                   mPackBwd.get() + (layer - 1) * kPackL, (const float *)nullptr, mAct[layer - 1].get(),
-		                   mG[1 - cur].get(), (const float *)nullptr, (float *)nullptr);
+		                   mG[1 - cur].get(), (const float *)nullptr, (float *)nullptr, zbricks);
 		cur = 1 - cur;
 	}
 	hipLaunchKernelGGL((k_conv_wgrad<4>), dim3(wg_blocks), dim3(256), 0, mStream, mNx, mNy, mNz, nbx, nby, nbz,

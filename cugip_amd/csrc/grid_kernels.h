@@ -17,7 +17,7 @@
 //               never run together (colour phases), so the only cross-tile write that needs an
 //               atomic is the excess of a halo voxel.
 //   * cut:      T_min = finite labels of the last exact relabel (fill_segments, graph_cut.hpp:304-333);
-//               S_min = closure of the excess voxels under residual edges (see DESIGN.md proof).
+//               S_min = closure of the excess voxels under residual edges (of a maximum preflow).
 #pragma once
 
 #include "common.h"

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void k_tile_tables(TileTables out, int32_t *__
 // when some edge's capacity pair exceeds 32767 (then residuals cannot be staged as int16).
 // Voxel-parallel over z-columns rather than tiles: the xy plane of a grid is cut into strips of
 // kInitThreads consecutive xy indices (x fastest, running on across rows, so no lane idles on a
-// partial tile), z into chunks of kInitDepth; workgroup b takes one strip × one chunk (strip-major
+// partial tile), z into chunks of kDepth levels; workgroup b takes one strip × one chunk (strip-major
 // within its chunk; block_inst / inst_first_block give the grid of b in a batch), thread t the
 // column of its xy index, whose +z neighbours are its own next voxels. 6C: all loads of a voxel are
 // issued before its arithmetic and stores; 26C: one residual plane at a time over the column.
@@ -150,12 +150,18 @@ __global__ __launch_bounds__(256) void k_tile_tables(TileTables out, int32_t *__
 // capacities a column's mirror residuals read (its 8 xy neighbours) mostly belong to the same
 // workgroup.
 constexpr int kInitThreads = 256, kInitDepth = 8, kInitTileX = 64, kInitTileY = kInitThreads / kInitTileX;
+// With fewer than kInitManyBlocks workgroups of kInitDepth levels, which leave the chip half empty, the chunks are
+// kInitDepthSmall deep: a workgroup is then a quarter of the instructions, and there are four times as many
+// to hide the loads. Init with 8 / 2 levels, 6-connected: 33 x 30 x 28 14.6 / 8 us, 98 x 96 x 91 26 / 15,
+// 160 x 160 x 160 (2000 workgroups of 8) 62 / 48, 194 x 190 x 157 (2880) 94 / 83, 256 x 256 x 256 (8192) 211 /
+// 214; 26-connected: 33 x 30 x 28 33 / 14 us, 77 x 71 x 64 55 / 28, 194 x 190 x 157 (3840) 370 / 345.
+constexpr int kInitDepthSmall = 2, kInitManyBlocks = 4096;
 
-__host__ __device__ inline int64_t init_blocks(int64_t nx, int64_t ny, int64_t nz, int conn)
+__host__ __device__ inline int64_t init_blocks(int64_t nx, int64_t ny, int64_t nz, int conn, int depth)
 {
 	const int64_t per_chunk = conn == 26 ? ((nx + kInitTileX - 1) / kInitTileX) * ((ny + kInitTileY - 1) / kInitTileY)
 	                                     : (nx * ny + kInitThreads - 1) / kInitThreads;
-	return per_chunk * ((nz + kInitDepth - 1) / kInitDepth);
+	return per_chunk * ((nz + depth - 1) / depth);
 }
 
 // Column (x, y) and z-chunk of thread threadIdx.x of init workgroup lb in the xy-tile layout.
@@ -177,12 +183,12 @@ __device__ inline void init_tile_coords(const GridView &g, int lb, int &x, int &
 // from the cache. Only one plane's address is live: voxel by voxel, all 39 plane addresses of a
 // 26-connected grid would stay live across the column, more than the scalar registers hold.
 // State bits and inflow sums stay in registers until the last plane.
-template <int kConn, bool kBack>
+template <int kConn, int kDepth, bool kBack>
 __device__ inline void init_column_by_plane(const GridView &g, int x, int y, int oz, uint32_t xy, uint32_t sxy,
                                             long long &cancelled, bool &negative, bool &overflow, bool &wide)
 {
 	using D = Dirs<kConn>;
-	constexpr int H = D::H, Z = kInitDepth;
+	constexpr int H = D::H, Z = kDepth;
 	// inflow sums saturate at 2^31 (each term is below 2^31, so the 32-bit sum cannot wrap): only
 	// whether one exceeds int32 matters; likewise a capacity pair's sum of two values below 2^31
 	uint32_t state[Z], incoming[Z];
@@ -268,7 +274,7 @@ __device__ inline void init_column_by_plane(const GridView &g, int x, int y, int
 	}
 }
 
-template <int kConn>
+template <int kConn, int kDepth>
 __global__ __launch_bounds__(kInitThreads) void k_grid_init(GridView gv, const int32_t *__restrict__ block_inst,
                                                            const int32_t *__restrict__ inst_first_block,
                                                            const SolveControl *ctl)
@@ -290,16 +296,16 @@ __global__ __launch_bounds__(kInitThreads) void k_grid_init(GridView gv, const i
 	long long cancelled = 0;
 	bool negative = false, overflow = false, wide = false;
 	// 6C: the whole column unrolled, voxel by voxel; 26C: plane by plane
-	constexpr int kUnroll = kInitDepth;
+	constexpr int kUnroll = kDepth;
 	if constexpr (kConn == 26) {
 		int x, y, chunk;
 		init_tile_coords(g, lb, x, y, chunk);
 		if (x < g.nx && y < g.ny) {
 			if (g.cnb) {
-				init_column_by_plane<kConn, true>(g, x, y, chunk * kInitDepth, slice_xy(g, x, y), sxy, cancelled,
+				init_column_by_plane<kConn, kDepth, true>(g, x, y, chunk * kDepth, slice_xy(g, x, y), sxy, cancelled,
 				                                  negative, overflow, wide);
 			} else {
-				init_column_by_plane<kConn, false>(g, x, y, chunk * kInitDepth, slice_xy(g, x, y), sxy, cancelled,
+				init_column_by_plane<kConn, kDepth, false>(g, x, y, chunk * kDepth, slice_xy(g, x, y), sxy, cancelled,
 				                                   negative, overflow, wide);
 			}
 		}
@@ -308,10 +314,10 @@ __global__ __launch_bounds__(kInitThreads) void k_grid_init(GridView gv, const i
 		const int chunk = lb / strips, strip = lb - chunk * strips;
 		const uint32_t xy = (uint32_t)strip * kInitThreads + threadIdx.x;
 		const int y = (int)(xy / (uint32_t)g.nx), x = (int)(xy - (uint32_t)y * (uint32_t)g.nx);
-		const int oz = chunk * kInitDepth;
+		const int oz = chunk * kDepth;
 		if (xy < sxy) {
 #pragma unroll kUnroll
-			for (int k = 0; k < kInitDepth; ++k) {
+			for (int k = 0; k < kDepth; ++k) {
 				const int z = oz + k;
 				if (z >= g.nz) {
 					continue;

@@ -563,9 +563,16 @@ void GridSolver::configure_tiles(const Shape &shape)
 	{
 		std::vector<int32_t> first(mInst.size());
 		int64_t blocks = 0;
-		for (size_t i = 0; i < mInst.size(); ++i) {
-			first[i] = (int32_t)blocks;
-			blocks += init_blocks(mInst[i].nx, mInst[i].ny, mInst[i].nz, mConn);
+		for (const int depth : {kInitDepth, kInitDepthSmall}) {
+			blocks = 0;
+			mInitDepth = depth;
+			for (size_t i = 0; i < mInst.size(); ++i) {
+				first[i] = (int32_t)blocks;
+				blocks += init_blocks(mInst[i].nx, mInst[i].ny, mInst[i].nz, mConn, depth);
+			}
+			if (blocks >= kInitManyBlocks) {
+				break;
+			}
 		}
 		mInitBlocks = (int)blocks;
 		if (batch) {
@@ -660,12 +667,14 @@ void GridSolver::launch_init(const SolveControl *ctl)
 		const bool batch = mInst.size() > 1;
 		const int32_t *block_inst = batch ? mInitBlockInst.get() : nullptr;
 		const int32_t *first = batch ? mInitFirstBlock.get() : nullptr;
+		const auto run = [&](auto kernel) {
+			hipLaunchKernelGGL(kernel, dim3(mInitBlocks), dim3(kInitThreads), 0, mStream, g, block_inst, first, ctl);
+		};
+		const bool deep = mInitDepth == kInitDepth;
 		if (mConn == 6) {
-			hipLaunchKernelGGL(k_grid_init<6>, dim3(mInitBlocks), dim3(kInitThreads), 0, mStream, g, block_inst, first,
-			                   ctl);
+			deep ? run(k_grid_init<6, kInitDepth>) : run(k_grid_init<6, kInitDepthSmall>);
 		} else {
-			hipLaunchKernelGGL(k_grid_init<26>, dim3(mInitBlocks), dim3(kInitThreads), 0, mStream, g, block_inst,
-			                   first, ctl);
+			deep ? run(k_grid_init<26, kInitDepth>) : run(k_grid_init<26, kInitDepthSmall>);
 		}
 	});
 }

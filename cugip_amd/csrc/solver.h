@@ -189,6 +189,7 @@ private:
 	DeviceBuffer<int32_t> mInitBlockInst;      // batches only: instance of every init workgroup
 	DeviceBuffer<int32_t> mInitFirstBlock;     // batches only: first init workgroup of every instance
 	int mInitBlocks = 0;
+	int mInitDepth = 0;  // z-levels of an init workgroup
 	// configure_tiles' tables are kept while the grids and the tile shape stay the same
 	bool mTilesReady = false;
 	Shape mReadyShape{0, 0, 0};

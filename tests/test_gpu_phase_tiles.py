@@ -1,6 +1,8 @@
-"""Discharge phases and sweeps on both sides of the tile count up to which they take their colour class
-whole instead of a compacted list, host-driven and (6-connected) device-driven: the flow equals the
-capacity of the cut it returns (integers, so the flow is maximum), and both engines give the same."""
+"""Where a grid's size changes the launches. Discharge phases and sweeps on both sides of the tile count
+up to which they take their colour class whole instead of a compacted list, host-driven and
+(6-connected) device-driven: the flow equals the capacity of the cut it returns (integers, so the flow
+is maximum), and both engines give the same. The init on both sides of the workgroup count that
+decides how many z-levels a workgroup takes."""
 import numpy as np
 import pytest
 
@@ -49,3 +51,18 @@ def test_phases_around_the_whole_colour_limit(conn, tile, across, extra):
         results.append((flow, inside))
     for flow, inside in results[1:]:
         assert flow == results[0][0] and np.array_equal(inside, results[0][1])
+
+
+@pytest.mark.parametrize("conn", [6, 26])
+@pytest.mark.parametrize("nz", [8 * 4095, 8 * 4095 + 1])
+def test_init_around_the_deep_chunk_limit(conn, nz):
+    # one strip (rectangle) of columns, 4095 and 4096 chunks of 8 levels
+    say(f"init of 9 x 3 x {nz}, {conn} connections")
+    rng = np.random.default_rng(conn)
+    cs, ct = (np.maximum(rng.integers(-300, 200, (nz, 3, 9)), 0).astype(np.int32) for _ in range(2))
+    cn = rng.integers(0, 60, (conn // 2, nz, 3, 9)).astype(np.int32)
+    with cugip_amd.GridGraph() as g:
+        g.set_grid(cs, ct, cn, conn=conn)
+        flow = g.max_flow()
+        inside = g.source_set().reshape(cs.shape).astype(bool)
+    assert flow == cut_capacity(cs, ct, cn, inside, conn)
